@@ -410,91 +410,6 @@ __global__ void w8a32_reference_kernel(const float* __restrict__ x,
     y[idx] = sum;
 }
 
-// Cooperative mode: bounded split-K.  Grid (ceil(N/64), M, P); partition p
-// covers the balanced K range [p*base + min(p, rem), ...); lane = column;
-// wave w accumulates k = begin + w, begin + w + 4, ... in order; the four
-// wave sums are added in fixed order ((w0 + w1) + w2) + w3.  P > 1 writes
-// partials that a second kernel adds in ascending p.  Deterministic.
-__global__ __launch_bounds__(kBlock) void w8a32_coop_kernel(
-    const float* __restrict__ x, const int8_t* __restrict__ q, float scale,
-    int32_t zp, float* __restrict__ out, int64_t rows, int64_t inner,
-    int64_t cols, int64_t parts) {
-    __shared__ float red[4][HM_WAVE];
-    const int lane = threadIdx.x & (HM_WAVE - 1);
-    const int wave = threadIdx.x / HM_WAVE;
-    const int64_t c = (int64_t)blockIdx.x * HM_WAVE + lane;
-    const int64_t r = blockIdx.y;
-    const int64_t p = blockIdx.z;
-    const int64_t base = inner / parts, rem = inner % parts;
-    const int64_t begin = p * base + (p < rem ? p : rem);
-    const int64_t end = begin + base + (p < rem ? 1 : 0);
-    float sum = 0.0f;
-    if (c < cols) {
-        for (int64_t k = begin + wave; k < end; k += 4) {
-            const float w = __fmul_rn((float)((int)q[k * cols + c] - zp), scale);
-            sum = __fadd_rn(sum, __fmul_rn(x[r * inner + k], w));
-        }
-    }
-    red[wave][lane] = sum;
-    __syncthreads();
-    if (wave == 0 && c < cols) {
-        const float s = __fadd_rn(__fadd_rn(__fadd_rn(red[0][lane], red[1][lane]), red[2][lane]),
-                                  red[3][lane]);
-        out[(p * rows + r) * cols + c] = s;
-    }
-}
-
-__global__ void reduce_parts_kernel(const float* __restrict__ parts_in, int64_t parts,
-                                    int64_t count, float* __restrict__ y) {
-    const int64_t idx = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (idx >= count) return;
-    float s = parts_in[idx];
-    for (int64_t p = 1; p < parts; ++p) s = __fadd_rn(s, parts_in[p * count + idx]);
-    y[idx] = s;
-}
-
-__global__ __launch_bounds__(kBlock) void matmul_f32_kernel(
-    const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ y,
-    int64_t rows, int64_t inner, int64_t cols) {
-    __shared__ float as[kF32K][kF32Tile + 1];
-    __shared__ float bs[kF32K][kF32Tile + 1];
-    const int tid = threadIdx.x;
-    const int64_t m0 = (int64_t)blockIdx.x * kF32Tile, n0 = (int64_t)blockIdx.y * kF32Tile;
-    const int tr = tid / 16, tc = tid % 16;
-    float acc[4][4] = {};
-    for (int64_t k0 = 0; k0 < inner; k0 += kF32K) {
-        for (int i = tid; i < kF32Tile * kF32K; i += kBlock) {
-            const int r = i / kF32K, kk = i % kF32K;
-            const int64_t k = k0 + kk;
-            as[kk][r] = (m0 + r < rows && k < inner) ? x[(m0 + r) * inner + k] : 0.0f;
-            const int kk2 = i / kF32Tile, cc = i % kF32Tile;
-            const int64_t k2 = k0 + kk2;
-            bs[kk2][cc] = (k2 < inner && n0 + cc < cols) ? w[k2 * cols + n0 + cc] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < kF32K; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = as[kk][tr + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = bs[kk][tc + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t r = m0 + tr + 16 * i, c = n0 + tc + 16 * j;
-            if (r < rows && c < cols) y[r * cols + c] = acc[i][j];
-        }
-}
-
 // [K x N] -> [N x K] transpose of one projection (32x32 LDS tiles).
 template <typename T>
 __global__ void transpose_kernel(const T* __restrict__ src, T* __restrict__ dst,
@@ -738,6 +653,11 @@ int hm_launch_down_f32_mfma(const hm_layer* L, const float* z, const int32_t* co
                             const int32_t* offsets, int64_t R, int64_t max_tiles, float* y,
                             hipStream_t stream);
 
+int hm_launch_op_gemm_f32(const float* x, const float* w, float* y, int64_t M, int64_t K, int64_t N,
+                          hipStream_t s);
+int hm_launch_op_gemm_w8a32(const float* x, const int8_t* q, float scale, int32_t zp, float* y,
+                            int64_t M, int64_t K, int64_t N, hipStream_t s);
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // FP32 experts: the matrix-core tiles (hm_gemm_f32_mfma.hip) where the
@@ -839,36 +759,20 @@ int hm_matmul_w8a32(const float* x, const int8_t* q, float scale, int32_t zp,
         HM_LAUNCHED();
         return HM_OK;
     }
+    // the cooperative plan: the matrix-core kernel (hm_op_gemm.hip) splits K
+    // over a workgroup's waves and needs no scratch; what the plan asks of
+    // the caller stays required
     if (rows > 65535) return HM_ERR_UNSUPPORTED;
-    const dim3 grid((unsigned)((cols + HM_WAVE - 1) / HM_WAVE), (unsigned)rows,
-                    (unsigned)plan.partitions);
-    if (plan.partitions == 1) {
-        hipLaunchKernelGGL(w8a32_coop_kernel, grid, dim3(kBlock), 0, s, x, q, scale, zp, y,
-                           rows, inner, cols, plan.partitions);
-        HM_LAUNCHED();
-        return HM_OK;
-    }
-    HM_REQUIRE(scratch && scratch_bytes >= (size_t)plan.scratch_elements * sizeof(float));
-    hipLaunchKernelGGL(w8a32_coop_kernel, grid, dim3(kBlock), 0, s, x, q, scale, zp, scratch,
-                       rows, inner, cols, plan.partitions);
-    HM_LAUNCHED();
-    const int64_t count = rows * cols;
-    hipLaunchKernelGGL(reduce_parts_kernel, dim3((unsigned)((count + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, s, scratch, plan.partitions, count, y);
-    HM_LAUNCHED();
-    return HM_OK;
+    HM_REQUIRE(plan.partitions == 1 ||
+               (scratch && scratch_bytes >= (size_t)plan.scratch_elements * sizeof(float)));
+    return hm_launch_op_gemm_w8a32(x, q, scale, zp, y, rows, inner, cols, s);
 }
 
 int hm_matmul_f32(const float* x, const float* w, float* y, int64_t rows, int64_t inner,
                   int64_t cols, void* stream) {
     HM_REQUIRE(x && w && y && rows > 0 && inner > 0 && cols > 0);
     HM_REQUIRE((const void*)x != (const void*)y && (const void*)w != (const void*)y);
-    const dim3 grid((unsigned)((rows + kF32Tile - 1) / kF32Tile),
-                    (unsigned)((cols + kF32Tile - 1) / kF32Tile));
-    hipLaunchKernelGGL(matmul_f32_kernel, grid, dim3(kBlock), 0, hm_stream(stream), x, w, y,
-                       rows, inner, cols);
-    HM_LAUNCHED();
-    return HM_OK;
+    return hm_launch_op_gemm_f32(x, w, y, rows, inner, cols, hm_stream(stream));
 }
 
 size_t hm_packed_layer_bytes(int64_t experts, int64_t hidden, int64_t intermediate,

@@ -165,15 +165,20 @@ int hm_gather_rows(const float* in, const int32_t* rows, int64_t count,
 /* ---- A5/A5' op level (TensorBackend::matmulInt8Weights / matmul,
  * src/tensor/backend/CpuTensorBackend.cpp:87-190).  x [M x K] FP32,
  * q / w [K x N] row-major INPUT_OUTPUT, y [M x N].
- * hm_matmul_w8a32 uses the reference's W8A32 arithmetic,
- * acc += x * (float(q - zp) * scale) in FP32, with a bounded deterministic
- * split-K (hm_plan_int8_gemm); within 1e-5 + 1e-5|ref| of the CPU path. */
+ * hm_matmul_w8a32, mode 1 (reference): the reference's loop,
+ * acc += x * (float(q - zp) * scale) in FP32, bit-exact.  Mode 2
+ * (cooperative): the terms x (q - zp) exactly, summed in FP32 in another,
+ * fixed order, times the scale; within 1e-5 + 1e-5|ref| of the CPU path.
+ * The plan (hm_plan_int8_gemm) is the reference's: its partition and block
+ * counts and the scratch it asks of the caller are part of the interface,
+ * though the cooperative kernel splits K inside a workgroup and leaves the
+ * scratch untouched. */
 typedef struct hm_int8_gemm_plan {
     int32_t implementation; /* 1 = Reference (one lane per output),
                                2 = Cooperative (split-K partitions) */
     int64_t partitions;     /* bounded split-K: min(8, ceil(K/512)) */
-    int64_t blocks;         /* workgroups launched */
-    int64_t scratch_elements; /* FP32 split-K scratch, M*N*P if P > 1 */
+    int64_t blocks;         /* workgroups of the reference's launch */
+    int64_t scratch_elements; /* FP32 scratch the call asks for, M*N*P if P > 1 */
 } hm_int8_gemm_plan;
 /* Launch plan, src/backend/cuda/Int8GemmPlan.cpp:29-53 (mode: 0 auto,
  * 1 reference, 2 cooperative). */

@@ -73,6 +73,82 @@ def test_w8a32_reference_inputs(dev, rows, inner, cols):
         assert np.all(np.abs(got - dbl) <= 1e-5 + 1e-5 * np.abs(cpu))
 
 
+# edges of the op-level kernels: 16-row and 32/64-column tiles, 16- and
+# 32-wide K steps, fewer K steps than waves, row counts that pick each tile
+OP_SHAPES = [(1, 1, 1), (1, 256, 64), (16, 31, 33), (17, 33, 31), (33, 257, 66), (65, 1000, 130),
+             (150, 768, 2048), (300, 2048, 768), (333, 519, 1027), (1200, 64, 2050)]
+
+
+def _op_call(dev, x, w, y, scale=None, zp=0):
+    rows, inner, cols = x.shape[0], x.shape[1], w.shape[1]
+    if scale is None:
+        dev.call("hm_matmul_f32", x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, inner, cols, dev.stream)
+        return
+    plan = capi.HmInt8GemmPlan()
+    capi.call("hm_plan_int8_gemm", rows, inner, cols, 2, C.byref(plan))
+    scratch = dev.empty(max(1, plan.scratch_elements), np.float32)
+    dev.call("hm_matmul_w8a32", x.data_ptr(), w.data_ptr(), scale, zp, y.data_ptr(), rows, inner, cols, 2,
+             scratch.data_ptr(), scratch.numel() * 4, dev.stream)
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("rows,inner,cols", OP_SHAPES)
+def test_op_gemm_edges(dev, rows, inner, cols, int8):
+    """The op-level products against 64-bit sums at the edges of their tiles and
+    K steps, from operands off their vector alignment: each output within
+    (K + 32) u sum |x w|, u = 2^-24 (K additions, at most 16 waves' sums and
+    the scale, each rounding once)."""
+    rng = np.random.default_rng(rows + inner + cols)
+    x = (rng.standard_normal((rows, inner)) * np.exp2(rng.integers(-12, 12, (rows, inner)))).astype(np.float32)
+    dx = dev.to(np.concatenate([np.zeros(1, np.float32), x.reshape(-1)]))[1:].view(rows, inner)
+    y = dev.empty((rows, cols), np.float32)
+    if int8:
+        zp, scale = (-128, 127, 0)[(rows + cols) % 3], float(np.float32(0.0031))
+        q = rng.integers(-128, 128, (inner, cols)).astype(np.int8)
+        dw = dev.to(np.concatenate([np.zeros(1, np.int8), q.reshape(-1)]))[1:].view(inner, cols)
+        _op_call(dev, dx, dw, y, scale, zp)
+        w = (q.astype(np.float64) - zp) * scale
+    else:
+        wf = rng.standard_normal((inner, cols)).astype(np.float32)
+        dw = dev.to(np.concatenate([np.zeros(1, np.float32), wf.reshape(-1)]))[1:].view(inner, cols)
+        _op_call(dev, dx, dw, y)
+        w = wf.astype(np.float64)
+    got = dev.host(y)
+    x64 = x.astype(np.float64)
+    assert np.all(np.abs(got - x64 @ w) <= (inner + 32) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w)))
+
+
+@pytest.mark.parametrize("int8", [True, False])
+def test_op_gemm_special_values(dev, int8):
+    """Non-finite operands reach exactly the outputs that the reference's loop
+    gives them (also in the last K step, past which the operands are zero), and
+    rows near the ends of the float range keep their 24 bits."""
+    M, K, N = 35, 301, 70
+    rng = np.random.default_rng(77)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[3, 5], x[4, 300], x[5, 7], x[33, 299] = np.inf, -np.inf, np.nan, np.inf
+    x[6], x[7] = x[6] * np.float32(2.0 ** -100), x[7] * np.float32(2.0 ** 100)
+    q = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    q[5, 9] = q[300, 11] = 0
+    wf = (q.astype(np.float32) * np.float32(0.01)).astype(np.float32)
+    if not int8:
+        wf[300, 13], wf[2, 14] = np.inf, np.nan
+    y = dev.empty((M, N), np.float32)
+    _op_call(dev, dev.to(x), dev.to(q if int8 else wf), y, 0.01 if int8 else None)
+    got = dev.host(y)
+    with np.errstate(all="ignore"):
+        ref = O.matmul_w8a32(x, q, 0.01, 0) if int8 else O.matmul_f32(x, wf)
+    fine = np.isfinite(ref)
+    assert_bitexact(np.isnan(got), np.isnan(ref), "NaN outputs")
+    inf = ~fine & ~np.isnan(ref)
+    assert_bitexact(got[inf], ref[inf], "infinite outputs")
+    x64, w64 = np.where(np.isfinite(x), x, 0).astype(np.float64), np.where(np.isfinite(wf), wf, 0).astype(np.float64)
+    bound = (K + 32) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64))
+    if int8:
+        w64 = q.astype(np.float64) * float(np.float32(0.01))
+    assert np.all(np.abs(got - x64 @ w64)[fine] <= bound[fine])
+
+
 def test_matmul_f32_closed_form(dev):
     """tests/phase5_tests.cpp:147-160: [[1,2,3],[4,5,6]] x [[7,8],[9,10],[11,12]]."""
     a = np.array([[1, 2, 3], [4, 5, 6]], np.float32)
