@@ -296,7 +296,8 @@ __device__ __forceinline__ float hm_recombine(const int* p, int limbs) {
 //   Z       [K64/64][L][R][64]    grouped rows: one plane's chunk of
 //                                 consecutive rows is contiguous (a 16-row
 //                                 load unit is one kilobyte)
-// Pad digits (K <= k < K64) are never read.
+// Pad digits (K <= k < K64; X and Z) are zeros where K is no multiple of 64:
+// the ring GEMMs read whole chunks.
 struct hm_dlay {
     int64_t row, plane, chunk;
 };
@@ -324,13 +325,15 @@ __host__ __device__ __forceinline__ int64_t hm_dlay_off(const hm_dlay& d, int l,
 // float4), its digit sum to dsum[l * dsum_stride] (when dsum is set), the
 // scale max|x| / range to *scale.  Shared by the row-quantisation kernels
 // and the routers' select kernels, so all of them write the same bytes.
+// RAG: the row is shorter than 256 nv (its values past the end are zeros in
+// v) and only the digits k < kend are stored.
 constexpr int kHmQuantMaxV = 16;  // n <= 4096
-template <int L>
+template <int L, bool RAG = false>
 __device__ __forceinline__ void hm_quantize_row_values(const float4* v, int nv,
                                                        int8_t* __restrict__ digits,
                                                        const hm_dlay& lay, float* scale,
                                                        int32_t* __restrict__ dsum,
-                                                       int64_t dsum_stride) {
+                                                       int64_t dsum_stride, int kend = 0) {
     const int lane = threadIdx.x & (HM_WAVE - 1);
     float amax = 0.0f;
 #pragma unroll
@@ -358,7 +361,8 @@ __device__ __forceinline__ void hm_quantize_row_values(const float4* v, int nv,
                 const uint32_t word = (uint32_t)(d0[l] & 255) | ((uint32_t)(d1[l] & 255) << 8) |
                                       ((uint32_t)(d2[l] & 255) << 16) | ((uint32_t)(d3[l] & 255) << 24);
                 const int64_t k = 4 * (int64_t)(lane + HM_WAVE * i);
-                *reinterpret_cast<uint32_t*>(digits + hm_dlay_off(lay, l, 0, k)) = word;
+                if (!RAG || k < kend)
+                    *reinterpret_cast<uint32_t*>(digits + hm_dlay_off(lay, l, 0, k)) = word;
                 dl[l] += d0[l] + d1[l] + d2[l] + d3[l];
             }
         }

@@ -24,11 +24,12 @@ constexpr int kBlock = 256;
 // ---------------------------------------------------------------------------
 // Activation rows -> digit planes (one wave per row segment).
 // digits in layout lay (hm_dlay: the op-level [L][rows][n] or the block's
-// X rows), scales [rows], dsum [L][rows].
+// X rows, whose pad digits n .. nend-1 become zeros; op level: nend = n),
+// scales [rows], dsum [L][rows].
 // ---------------------------------------------------------------------------
 template <int L>
 __global__ __launch_bounds__(kBlock) void limb_quantize_rows_kernel(
-    const float* __restrict__ x, int64_t rows, int64_t n,
+    const float* __restrict__ x, int64_t rows, int64_t n, int64_t nend,
     int8_t* __restrict__ digits, hm_dlay lay, float* __restrict__ scales,
     int32_t* __restrict__ dsum) {
     const int lane = threadIdx.x & (HM_WAVE - 1);
@@ -52,6 +53,9 @@ __global__ __launch_bounds__(kBlock) void limb_quantize_rows_kernel(
             dl[l] += d;
         }
     }
+    if (n + lane < nend)
+#pragma unroll
+        for (int l = 0; l < L; ++l) digits[hm_dlay_off(lay, l, r, n + lane)] = 0;
 #pragma unroll
     for (int l = 0; l < L; ++l) {
         const int s = hm_wave_sum_i32(dl[l]);
@@ -85,10 +89,11 @@ __global__ __launch_bounds__(kBlock) void limb_quantize_rows_vec_kernel(
 // like any activation row (one scale per row).  One wave per row.  Digits
 // in the Z layout (hm_dlay_z(L, rows)).
 // ---------------------------------------------------------------------------
-// rows of n = 256 * NV, 16-byte aligned: the row in registers (NV a
-// template argument, so a wave holds only its own row's values)
-template <int L, int NV>
-__global__ __launch_bounds__(kBlock) void limb_swiglu_quantize_vec_kernel(
+// rows of n = 256 * NV (RAG: any multiple of 4 up to that), 16-byte
+// aligned: the row in registers (NV a template argument, so a wave holds only
+// its own row's values; RAG: zeros past n, whose digits are the pad's zeros)
+template <int L, int NV, bool RAG>
+__device__ __forceinline__ void limb_swiglu_quantize_row(
     const float* __restrict__ gu, int64_t rows, int64_t n,
     int8_t* __restrict__ digits, float* __restrict__ scales, int32_t* __restrict__ dsum) {
     __shared__ unsigned long long s_exp2[32];
@@ -102,8 +107,16 @@ __global__ __launch_bounds__(kBlock) void limb_swiglu_quantize_vec_kernel(
     float4 g[NV], u[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        g[i] = g4[lane + HM_WAVE * i];
-        u[i] = u4[lane + HM_WAVE * i];
+        const int q = lane + HM_WAVE * i;
+        if constexpr (RAG) {
+            const int qc = min(q, (int)(n / 4) - 1);
+            g[i] = g4[qc];
+            u[i] = u4[qc];
+            if (q != qc) g[i] = u[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        } else {
+            g[i] = g4[q];
+            u[i] = u4[q];
+        }
     }
     bool small = true;
 #pragma unroll
@@ -131,8 +144,20 @@ __global__ __launch_bounds__(kBlock) void limb_swiglu_quantize_vec_kernel(
         }
     }
     const hm_dlay lay = hm_dlay_z(L, rows);
-    hm_quantize_row_values<L>(z, NV, digits + r * lay.row, lay, scales + r,
-                              dsum ? dsum + r : nullptr, rows);
+    hm_quantize_row_values<L, RAG>(z, NV, digits + r * lay.row, lay, scales + r,
+                                   dsum ? dsum + r : nullptr, rows, (int)hm_pad64(n));
+}
+template <int L, int NV>
+__global__ __launch_bounds__(kBlock) void limb_swiglu_quantize_vec_kernel(
+    const float* __restrict__ gu, int64_t rows, int64_t n,
+    int8_t* __restrict__ digits, float* __restrict__ scales, int32_t* __restrict__ dsum) {
+    limb_swiglu_quantize_row<L, NV, false>(gu, rows, n, digits, scales, dsum);
+}
+template <int L, int NV>
+__global__ __launch_bounds__(kBlock) void limb_swiglu_quantize_ragged_kernel(
+    const float* __restrict__ gu, int64_t rows, int64_t n,
+    int8_t* __restrict__ digits, float* __restrict__ scales, int32_t* __restrict__ dsum) {
+    limb_swiglu_quantize_row<L, NV, true>(gu, rows, n, digits, scales, dsum);
 }
 
 // any n: z recomputed in the digit pass
@@ -167,6 +192,9 @@ __global__ __launch_bounds__(kBlock) void limb_swiglu_quantize_kernel(
             dl[l] += d;
         }
     }
+    if (n + lane < hm_pad64(n))
+#pragma unroll
+        for (int l = 0; l < L; ++l) digits[hm_dlay_off(hm_dlay_z(L, rows), l, r, n + lane)] = 0;
 #pragma unroll
     for (int l = 0; l < L; ++l) {
         const int sm = hm_wave_sum_i32(dl[l]);
@@ -470,8 +498,8 @@ __global__ __launch_bounds__(256) void pack_tiles_i8_kernel(const int8_t* __rest
 // ===========================================================================
 // Launchers used by the block entry (hm_block.hip) and the C ABI.
 // ===========================================================================
-// Rows -> digit planes.
-static int quantize_rows(const float* x, int64_t rows, int64_t n, int32_t limbs,
+// Rows -> digit planes (pad digits n .. nend-1 zeroed).
+static int quantize_rows(const float* x, int64_t rows, int64_t n, int64_t nend, int32_t limbs,
                          int8_t* digits, const hm_dlay& lay, float* scales, int32_t* dsum,
                          hipStream_t stream) {
     if (rows == 0) return HM_OK;
@@ -491,7 +519,7 @@ static int quantize_rows(const float* x, int64_t rows, int64_t n, int32_t limbs,
         return HM_OK;
     }
 #define HM_QS(LV) HM_STAGE_LAUNCH(false, false, limb_quantize_rows_kernel<LV>, grid, dim3(kBlock), 0, stream, \
-                                  x, rows, n, digits, lay, scales, dsum)
+                                  x, rows, n, nend, digits, lay, scales, dsum)
     switch (limbs) {
     case 1: HM_QS(1); break;
     case 2: HM_QS(2); break;
@@ -507,7 +535,8 @@ static int quantize_rows(const float* x, int64_t rows, int64_t n, int32_t limbs,
 int hm_launch_quantize_rows(const float* x, int64_t rows, int64_t n, int32_t limbs,
                             int8_t* digits, float* scales, int32_t* dsum,
                             hipStream_t stream) {
-    return quantize_rows(x, rows, n, limbs, digits, hm_dlay_x(limbs, n), scales, dsum, stream);
+    return quantize_rows(x, rows, n, hm_pad64(n), limbs, digits, hm_dlay_x(limbs, n), scales, dsum,
+                         stream);
 }
 
 // gu [rows x 2n] (g | u per row) -> z = silu(g) * u -> digit planes in the
@@ -520,7 +549,8 @@ static int swiglu_quantize_rows(const float* gu, int64_t rows, int64_t n, int32_
     if (limbs < 1 || limbs > 3) return HM_ERR_INVALID;
     const dim3 grid((unsigned)((rows + 3) / 4));
     const int64_t nv = n / 256;
-    const bool vec = n % 256 == 0 && (uintptr_t)gu % 16 == 0 && (uintptr_t)digits % 4 == 0;
+    const bool vec4 = n % 4 == 0 && (uintptr_t)gu % 16 == 0 && (uintptr_t)digits % 4 == 0;
+    const bool vec = vec4 && n % 256 == 0;
 #define HM_SQ(LV, NV) HM_STAGE_LAUNCH(false, true, (limb_swiglu_quantize_vec_kernel<LV, NV>), grid, \
                                       dim3(kBlock), 0, stream, gu, rows, n, digits, scales, dsum)
 #define HM_SQL(NV)                                          \
@@ -535,6 +565,15 @@ static int swiglu_quantize_rows(const float* gu, int64_t rows, int64_t n, int32_
     else if (vec && nv == 4) HM_SQL(4);
     else if (vec && nv == 6) HM_SQL(6);
     else if (vec && nv == 8) HM_SQL(8);
+#undef HM_SQ
+#define HM_SQ(LV, NV) HM_STAGE_LAUNCH(false, true, (limb_swiglu_quantize_ragged_kernel<LV, NV>), grid, \
+                                      dim3(kBlock), 0, stream, gu, rows, n, digits, scales, dsum)
+    // other multiples of 4 (16-byte rows) up to 2048, on the next of these sizes
+    else if (vec4 && n <= 512) HM_SQL(2);
+    else if (vec4 && n <= 768) HM_SQL(3);
+    else if (vec4 && n <= 1024) HM_SQL(4);
+    else if (vec4 && n <= 1536) HM_SQL(6);
+    else if (vec4 && n <= 2048) HM_SQL(8);
     else {
 #define HM_SG(LV) HM_STAGE_LAUNCH(false, true, limb_swiglu_quantize_kernel<LV>, grid, dim3(kBlock), 0, \
                                   stream, gu, rows, n, digits, scales, dsum)
@@ -697,7 +736,7 @@ int hm_limb_quantize_rows(const float* x, int64_t rows, int64_t inner, int32_t l
                           int8_t* digits, float* scales, void* stream) {
     HM_REQUIRE(x && digits && scales && rows >= 0 && inner > 0);
     HM_REQUIRE(limbs >= 1 && limbs <= 3);
-    return quantize_rows(x, rows, inner, limbs, digits, hm_dlay_planes(rows, inner), scales,
+    return quantize_rows(x, rows, inner, inner, limbs, digits, hm_dlay_planes(rows, inner), scales,
                          nullptr, hm_stream(stream));
 }
 

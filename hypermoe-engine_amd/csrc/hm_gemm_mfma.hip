@@ -20,6 +20,7 @@
 //            (the SwiGLU runs in the Z quantisation pass, hm_gemm.hip).
 //   ring_gemm_kernel<L, true> (down): the same kernel on the grouped rows'
 //            Z digit planes and the down tiles; epilogue y -> floats.
+//   ring_gemm_ragged_kernel: both for shapes off the tile grid.
 //   limb_gemm_kernel (down, for shapes the ring does not take): 4 wave64s
 //            (one per SIMD, 512 registers: the accumulators take the
 //            AGPRs), A through an LDS ring by DMA, B straight into a
@@ -879,8 +880,17 @@ struct GateUpTile {
 // grouped rows themselves (a 16-row load unit is one contiguous kilobyte),
 // out = y [R x H] (tile: 256 down columns; the "gate" half of the gate/up
 // tile is its first 128 columns, the "up" half the next).
-template <int L, bool DN>
-__global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
+// RAG = true: shapes off the tile grid, with the same integers and floats.
+// K is walked in whole 64-byte chunks: the digits past K are zeros (the
+// quantisers write them), and where the weights' last 32-wide tile is the
+// first half of a stage, its second half re-reads that tile (against zero
+// digits).  Column blocks past the last re-read it, and columns past N are
+// not stored.  A form of its own so that the aligned shapes keep their loop
+// and registers.  The generic kernels (one lane per output, byte loads) took
+// such shapes before: 201 tokens, 60 experts top-4, H = 1024, I = 704: the
+// whole block 2778 -> 150 us.
+template <int L, bool DN, bool RAG>
+__device__ __forceinline__ void ring_gemm_body(
     const int8_t* __restrict__ xdig, const float* __restrict__ xscale,
     const int32_t* __restrict__ xdsum, int tokens, int H, int I, int experts,
     const int8_t* __restrict__ packed, const float* __restrict__ scale,
@@ -890,7 +900,7 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
     using T = GateUpTile<L>;
     // inner and output dimensions of the projection(s), output columns per
     // tile, the out row stride and the offset of the tile's second half
-    const int K = DN ? I : H, N = DN ? H : I;
+    const int K = RAG ? (int)hm_pad64(DN ? I : H) : (DN ? I : H), N = DN ? H : I;
     constexpr int TN = DN ? 2 * kGuN : kGuN;
     const int64_t ldo = DN ? (int64_t)N : 2 * (int64_t)N;
     const int half = DN ? kGuN : N;
@@ -923,11 +933,14 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
     __syncthreads();
     if (wave == 0) tile_prefix(s_cnt, E, BM, skinny, s_prefix);
     __syncthreads();
-    const int nbn = N / TN;
+    const int nbn = RAG ? (N + TN - 1) / TN : N / TN;
     const TileRange tr = tile_range(s_prefix[E] * nbn);
     if (tr.ntiles == 0) return;
     const int nk = K / kGuKB;
-    const int64_t tiles_k = hm_pad32(K) / 32;  // K tiles of one 32-column block
+    const int64_t tiles_k = hm_pad32(DN ? I : H) / 32;  // K tiles of one 32-column block
+    const int last_cb = (int)(hm_pad32(N) / 32) - 1;    // (RAG)
+    // (RAG) the stage whose second K half has no tile of its own
+    const int odd_ks = (tiles_k & 1) ? nk - 1 : -1;
 
     auto info = [&](int i) __attribute__((always_inline)) {
         const int j = tr.jbeg + i * tr.step;
@@ -998,19 +1011,29 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
                 }
             } else {
                 const int fb = f - NA;
-                const int64_t cb = t.n0 / 32 + (DN ? fb : (fb & 3));
+                int cb = t.n0 / 32 + (DN ? fb : (fb & 3));
+                if constexpr (RAG) cb = min(cb, last_cb);
                 src[c] = packed + hm_proj_offset(t.e, DN ? 2 : fb >> 2, H, I) +
-                         (cb * tiles_k + h) * 1024 + 16 * lane;
+                         ((int64_t)cb * tiles_k + h) * 1024 + 16 * lane;
             }
         }
     };
     // load c of a stage exists on this wave
     auto has_unit = [&](int c) __attribute__((always_inline)) { return c < LPW - 1 || full; };
+    // where load c of stage ks starts
+    auto stage_src = [&](const int8_t* const (&src)[LPW], int c, int ks) __attribute__((always_inline)) {
+        int64_t o = (int64_t)ks * sstep[c];
+        if constexpr (RAG) {
+            const int u = (wave + kGuWaves * c) % NL;
+            if (ks == odd_ks && (u >> 1) >= NA && (u & 1)) o -= 1024;
+        }
+        return src[c] + o;
+    };
     auto issue = [&](int slot, const int8_t* const (&src)[LPW], int ks) {
         int8_t* st = ring + slot * STAGE;
 #pragma unroll
         for (int c = 0; c < LPW; ++c)
-            if (has_unit(c)) dma16(src[c] + (int64_t)ks * sstep[c], st + dst[c]);
+            if (has_unit(c)) dma16(stage_src(src, c, ks), st + dst[c]);
     };
     // wait until at most n stages of this wave's loads are in flight
     auto vm_wait_stages = [&](auto nst) __attribute__((always_inline)) {
@@ -1068,7 +1091,7 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
             else
                 acc[ii][l][j] = mfma32(fa[h][ii][l], fb[h][j], acc[ii][l][j]);
             if (h == 0 && mi < LPW && dslot >= 0 && has_unit(mi))
-                dma16(src[mi] + (int64_t)dks * sstep[mi], ring + dslot * STAGE + dst[mi]);
+                dma16(stage_src(src, mi, dks), ring + dslot * STAGE + dst[mi]);
             if (rslot >= 0) {
                 if (j == NJ - 1) read_a(rslot, h, ii, l);
                 if (ii == WR - 1 && l == L - 1) read_b(rslot, h, j);
@@ -1078,7 +1101,7 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
         if (h == 0 && dslot >= 0)
 #pragma unroll
             for (int c = NM; c < LPW; ++c)
-                if (has_unit(c)) dma16(src[c] + (int64_t)dks * sstep[c], ring + dslot * STAGE + dst[c]);
+                if (has_unit(c)) dma16(stage_src(src, c, dks), ring + dslot * STAGE + dst[c]);
     };
     auto read_all = [&](int slot) __attribute__((always_inline)) {
 #pragma unroll
@@ -1169,6 +1192,7 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
             const int e = cur.e, nrows = cur.nrows;
             const float sg = s_sg[e], su = s_su[e];
             const int zg = s_zg[e], zu = s_zu[e];
+            const int col = cur.n0 + 32 * wc * WCP + (lane & 31);  // (RAG) the lane's column
 #pragma unroll
             for (int ii = 0; ii < WR; ++ii) {
                 const int r0 = 32 * (wr * WR + ii);
@@ -1207,7 +1231,12 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
                             }
                             const float g = __fmul_rn(hm_recombine(pg, L), fg);
                             const float u = __fmul_rn(hm_recombine(pu, L), fu);
-                            if (live) {
+                            if constexpr (RAG) {
+                                if (live && col + 32 * j < N) {
+                                    grow[32 * j] = g;
+                                    if (!DN || col + kGuN + 32 * j < N) grow[half + 32 * j] = u;
+                                }
+                            } else if (live) {
                                 if constexpr (DN) {
                                     grow[32 * j] = g;
                                     grow[half + 32 * j] = u;
@@ -1235,18 +1264,38 @@ __global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
     }
 }
 
-bool gateup_shape_ok(int64_t H, int64_t I, int64_t E, int32_t limbs) {
-    // |P_l| <= H * 128 * 255 < 2^31 keeps every limb partial exact: H <= 65536
-    return limbs >= 1 && limbs <= 3 && E >= 1 && E <= kMaxExperts && H <= 65536 &&
-           I <= (1 << 20) && H % kGuKB == 0 && H / kGuKB >= kGuStages && I % kGuN == 0;
+template <int L, bool DN>
+__global__ __launch_bounds__(kGuThreads) void ring_gemm_kernel(
+    const int8_t* __restrict__ xdig, const float* __restrict__ xscale,
+    const int32_t* __restrict__ xdsum, int tokens, int H, int I, int experts,
+    const int8_t* __restrict__ packed, const float* __restrict__ scale,
+    const int32_t* __restrict__ zp, const int32_t* __restrict__ counts,
+    const int32_t* __restrict__ offsets, const int32_t* __restrict__ perm_tokens, int skinny,
+    float* __restrict__ gu) {
+    ring_gemm_body<L, DN, false>(xdig, xscale, xdsum, tokens, H, I, experts, packed, scale, zp, counts, offsets, perm_tokens,
+                                    skinny, gu);
 }
 
-// The down projection on the ring kernel: K = I in 64-byte stages, N = H in
-// 256-column tiles.
-bool down_ring_ok(int64_t H, int64_t I, int64_t E, int32_t limbs) {
-    return limbs >= 1 && limbs <= 3 && E >= 1 && E <= kMaxExperts && I <= 65536 &&
-           H <= (1 << 20) && I % kGuKB == 0 && I / kGuKB >= kGuStages && H % (2 * kGuN) == 0;
+template <int L, bool DN>
+__global__ __launch_bounds__(kGuThreads) void ring_gemm_ragged_kernel(
+    const int8_t* __restrict__ xdig, const float* __restrict__ xscale,
+    const int32_t* __restrict__ xdsum, int tokens, int H, int I, int experts,
+    const int8_t* __restrict__ packed, const float* __restrict__ scale,
+    const int32_t* __restrict__ zp, const int32_t* __restrict__ counts,
+    const int32_t* __restrict__ offsets, const int32_t* __restrict__ perm_tokens, int skinny,
+    float* __restrict__ gu) {
+    ring_gemm_body<L, DN, true>(xdig, xscale, xdsum, tokens, H, I, experts, packed, scale, zp, counts, offsets, perm_tokens,
+                                    skinny, gu);
 }
+
+// Shapes of the ring kernel: K in at least kGuStages 64-byte stages.
+bool ring_ok(int64_t K, int64_t N, int64_t E, int32_t limbs) {
+    // |P_l| <= K * 128 * 255 < 2^31 keeps every limb partial exact: K <= 65536
+    return limbs >= 1 && limbs <= 3 && E >= 1 && E <= kMaxExperts && K <= 65536 &&
+           N <= (1 << 20) && hm_pad64(K) / kGuKB >= kGuStages;
+}
+// ... on its tile grid: whole stages and whole column blocks.
+bool ring_aligned(int64_t K, int64_t N, int64_t cols) { return K % kGuKB == 0 && N % cols == 0; }
 
 // Down: skinny groups (split K, when asked for), then the tiles of the
 // others on the ring kernel, or on limb_gemm_kernel where the ring's shape
@@ -1255,7 +1304,7 @@ template <int L>
 int launch_down(const hm_layer* layer, const int8_t* zdig, const float* zscale,
                 const int32_t* zdsum, int64_t R, const int32_t* counts, const int32_t* offsets,
                 float* y, bool split_k, hipStream_t stream) {
-    if (!down_ring_ok(layer->hidden, layer->intermediate, layer->experts, L))
+    if (!ring_ok(layer->intermediate, layer->hidden, layer->experts, L))
         return launch_l<L>(layer, zdig, zscale, zdsum, R, counts, offsets, y, split_k, stream);
     const bool sk = split_k && skinny_ok(layer->intermediate, layer->hidden, L, false);
     if (sk) {
@@ -1263,11 +1312,15 @@ int launch_down(const hm_layer* layer, const int8_t* zdig, const float* zscale,
                                                offsets, y, stream, false);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL((ring_gemm_kernel<L, true>), dim3((unsigned)persistent_grid()),
-                       dim3(kGuThreads), 0, stream, zdig, zscale, zdsum, (int)R,
-                       (int)layer->hidden, (int)layer->intermediate, (int)layer->experts,
-                       static_cast<const int8_t*>(layer->packed), layer->scale,
-                       layer->zero_point, counts, offsets, nullptr, sk ? kSkinnyRows : 0, y);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)persistent_grid()), dim3(kGuThreads), 0, stream,
+                           zdig, zscale, zdsum, (int)R, (int)layer->hidden,
+                           (int)layer->intermediate, (int)layer->experts,
+                           static_cast<const int8_t*>(layer->packed), layer->scale,
+                           layer->zero_point, counts, offsets, nullptr, sk ? kSkinnyRows : 0, y);
+    };
+    if (ring_aligned(layer->intermediate, layer->hidden, 2 * kGuN)) run(ring_gemm_kernel<L, true>);
+    else run(ring_gemm_ragged_kernel<L, true>);
     HM_LAUNCHED();
     return HM_OK;
 }
@@ -1285,26 +1338,29 @@ int launch_gateup(const hm_layer* layer, const int8_t* xdig, const float* xscale
                                               counts, offsets, gu, stream, true);
         if (rc) return rc;
     }
-    HM_STAGE_LAUNCH(!sk, false, (ring_gemm_kernel<L, false>), dim3((unsigned)persistent_grid()),
-                    dim3(kGuThreads), 0, stream, xdig, xscale, xdsum, (int)tokens,
-                    (int)layer->hidden, (int)layer->intermediate, (int)layer->experts,
-                    static_cast<const int8_t*>(layer->packed), layer->scale, layer->zero_point,
-                    counts, offsets, perm_tokens, sk ? kSkinnyRows : 0, gu);
+    auto run = [&](auto kernel) {
+        HM_STAGE_LAUNCH(!sk, false, kernel, dim3((unsigned)persistent_grid()), dim3(kGuThreads), 0,
+                        stream, xdig, xscale, xdsum, (int)tokens, (int)layer->hidden,
+                        (int)layer->intermediate, (int)layer->experts,
+                        static_cast<const int8_t*>(layer->packed), layer->scale,
+                        layer->zero_point, counts, offsets, perm_tokens, sk ? kSkinnyRows : 0, gu);
+    };
+    if (ring_aligned(layer->hidden, layer->intermediate, kGuN)) run(ring_gemm_kernel<L, false>);
+    else run(ring_gemm_ragged_kernel<L, false>);
     HM_LAUNCHED();
     return HM_OK;
 }
 
 }  // namespace
 
-// Shape preconditions of the MFMA kernels: K in 128-byte stages (enough of
-// them for the stream's look-ahead, a count the B register ring divides),
-// N in whole workgroup column blocks, E <= 256 (tables in LDS).
+// Shape preconditions of the MFMA kernels: at least four 64-byte K stages
+// (the ring's look-ahead), E <= 256 (tables in LDS), any N.
 bool hm_mfma_gateup_ok(int64_t H, int64_t I, int64_t E, int32_t limbs) {
-    return gateup_shape_ok(H, I, E, limbs);
+    return ring_ok(H, I, E, limbs);
 }
 
 bool hm_mfma_down_ok(int64_t H, int64_t I, int64_t E, int32_t limbs) {
-    return down_ring_ok(H, I, E, limbs) || shape_ok(I, H, E, limbs);
+    return ring_ok(I, H, E, limbs) || shape_ok(I, H, E, limbs);
 }
 
 // gu [R x 2I]: the gate and up values of every grouped row (X digits in the

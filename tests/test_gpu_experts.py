@@ -225,6 +225,38 @@ BLOCK_CASES = [  # (T, H, E, I, k, X digits, Z digits) -- MFMA shapes and generi
     (160, 2048, 64, 768, 8, 2, 3), (160, 512, 64, 256, 8, 2, 2)]
 
 
+# shapes off the ring kernel's tile grid: K with one or two 32-wide tiles in
+# its last 64-byte stage, exactly four stages, fewer columns than a tile,
+# ragged last column blocks, widths off 4 (the scalar SwiGLU) and past 2048
+RAGGED_CASES = [
+    (70, 1024, 60, 704, 4, 2, 3), (45, 320, 5, 272, 2, 3, 2), (150, 448, 9, 336, 3, 2, 3),
+    (40, 225, 4, 1000, 2, 1, 3), (33, 608, 6, 450, 3, 2, 1), (130, 256, 3, 2052, 2, 2, 3),
+    (90, 200, 4, 198, 2, 2, 2)]
+
+
+@pytest.mark.parametrize("T,H,E,I,k,LX,LZ", RAGGED_CASES)
+def test_block_int8_ragged_tiles(dev, T, H, E, I, k, LX, LZ):
+    """Shapes off the tile grid run the ring kernels too: the same bits as the
+    limb oracle, as the generic kernels (what they ran before), and with the
+    split-K kernel taking the small groups; zero points other than zero, and a
+    workspace full of other values (pad digits must come from the quantisers)."""
+    print(f"[gpu] ragged int8 T={T} H={H} E={E} I={I} k={k} limbs=({LX}, {LZ})", flush=True)
+    payload, scale, zp, h, w = _layer_inputs(61 + T, T, H, E, I, True)
+    zp = np.random.default_rng(T).integers(-20, 21, zp.shape).astype(np.int32)
+    block = MoEBlock(DeviceExpertLayer(payload, scale, zp, H, I), k, limbs_x=LX, limbs_z=LZ)
+    block.execute_batch(dev.to(h), dev.to(w), exec_flags=capi.HM_EXEC_LIMBS)
+    block._ws.fill_(0x55)
+    res = block.execute_batch(dev.to(h), dev.to(w), exec_flags=capi.HM_EXEC_LIMBS)
+    out = dev.host(res.output)
+    lout, lids, _ = O.moe_block_limbs(payload, scale, zp, h, w, k, I, LX, LZ)
+    assert_bitexact(res.ids, lids, "ids")
+    assert_bitexact(out, lout, "block output vs limb oracle")
+    for flags in (capi.HM_EXEC_GENERIC, capi.HM_EXEC_LIMBS | capi.HM_EXEC_SPLIT_K):
+        other = block.execute_batch(dev.to(h), dev.to(w), exec_flags=flags)
+        assert_bitexact(dev.host(other.output), out, f"exec flags {flags:#x}")
+        assert_bitexact(dev.host(other.expert_out), dev.host(res.expert_out), f"expert rows, flags {flags:#x}")
+
+
 @pytest.mark.parametrize("T,H,E,I,k,LX,LZ", BLOCK_CASES)
 def test_block_int8_bitexact_vs_limb_oracle(dev, T, H, E, I, k, LX, LZ):
     print(f"[gpu] block int8 T={T} H={H} E={E} I={I} k={k} limbs=({LX}, {LZ})", flush=True)
