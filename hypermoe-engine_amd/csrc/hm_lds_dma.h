@@ -61,4 +61,15 @@ __device__ __forceinline__ void dma4(const void* gsrc, void* lds_base) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off"
                  :: "v"(gsrc), "s"(m0) : "memory", "m0");
 }
+// dma16 and dma4 from a uniform base plus a 32-bit byte offset per lane.
+__device__ __forceinline__ void dma16_off(const void* base, uint32_t off, void* lds_base) {
+    const unsigned m0 = (unsigned)(uintptr_t)(lds_ptr_t)lds_base;
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(off), "s"(base), "s"(m0) : "memory", "m0");
+}
+__device__ __forceinline__ void dma4_off(const void* base, uint32_t off, void* lds_base) {
+    const unsigned m0 = (unsigned)(uintptr_t)(lds_ptr_t)lds_base;
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+                 :: "v"(off), "s"(base), "s"(m0) : "memory", "m0");
+}
 #pragma clang diagnostic pop

@@ -29,7 +29,7 @@ __device__ __forceinline__ void hm_status_or(int32_t* status, unsigned bits) {
 // inv(s) = 1/sqrt(s/W + eps) and y(inv) = float(x * inv * g) are monotone
 // under IEEE rounding, so an element whose y is equal at both ends of the
 // interval equals the reference's y.  If any element of the row is
-// ambiguous, the row falls back to the sequential sum (thread 0), which is
+// ambiguous, the row falls back to the sequential sum (one wave), which is
 // the reference computation itself.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double hm_inv_rms(double s, double width, double eps) {
@@ -44,21 +44,56 @@ __device__ __forceinline__ double hm_rms_sum_slack(int64_t width) {
     return 4.0 * gam / (1.0 - gam);
 }
 
-// The reference's own sum: double(x_k)^2 added in ascending k from +0
-// (the values read 16 at a time, so that the reads overlap the additions).
-__device__ __forceinline__ double hm_rms_sum_seq(const float* __restrict__ xr, int64_t width) {
+// Sequential FP64 chains.  The references' sums are chains of dependent
+// additions s_k = fl(s_{k-1} + p_k), and a dependent FP64 addition takes nine
+// cycles here whatever feeds it, so what a chain costs on top is how its terms
+// reach it.  They come through DPP: the 16 lanes of a row hold 64 consecutive
+// terms, lane i the terms 4 i .. 4 i + 3, and each step is one v_fmac_f64
+// whose first operand is lane i's term broadcast over the row
+// (row_newbcast:i; times 1.0, so the one rounding is the addition's): 9.3
+// cycles a step and no LDS round trip, register move or wait between steps.
+// Each row of 16 lanes runs a chain of its own (four chains a wave; with the
+// same terms in every row, every lane gets the sum).  All lanes of the wave
+// must be active.  (The leading s_nop covers the DPP read of a register that
+// the instruction before the block wrote.)
+#define HM_CHAIN4(i)                                                                \
+    "v_fmac_f64_dpp %0, %1, %5 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %0, %2, %5 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %0, %3, %5 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %0, %4, %5 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void hm_chain64(double& acc, double p0, double p1, double p2, double p3) {
+    asm volatile("s_nop 4\n\t"
+                 HM_CHAIN4(0) HM_CHAIN4(1) HM_CHAIN4(2) HM_CHAIN4(3) HM_CHAIN4(4) HM_CHAIN4(5)
+                 HM_CHAIN4(6) HM_CHAIN4(7) HM_CHAIN4(8) HM_CHAIN4(9) HM_CHAIN4(10) HM_CHAIN4(11)
+                 HM_CHAIN4(12) HM_CHAIN4(13) HM_CHAIN4(14) HM_CHAIN4(15)
+                 : "+v"(acc)
+                 : "v"(p0), "v"(p1), "v"(p2), "v"(p3), "v"(1.0));
+}
+#undef HM_CHAIN4
+
+// The reference's own sum of squares: double(x_k)^2 added in ascending k from
+// +0 (terms past the end are +0, which changes no sum of squares).  Every
+// lane returns it; xr in LDS or global memory.
+__device__ __forceinline__ double hm_rms_sum_seq(const float* xr, int64_t width) {
+    const int64_t i = 4 * (threadIdx.x & 15);
+    const int64_t last = width - 1;
+    auto load = [&](int64_t k0, float (&v)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int64_t k = k0 + i + q;
+            v[q] = xr[k < last ? k : last];
+            if (k > last) v[q] = 0.0f;
+        }
+    };
     double s = 0.0;
-    int64_t i = 0;
-    for (; i + 16 <= width; i += 16) {
-        float r[16];
+    float cur[4], nxt[4];
+    load(0, cur);
+    for (int64_t k0 = 0; k0 < width; k0 += 64) {
+        load(k0 + 64, nxt);
+        hm_chain64(s, (double)cur[0] * cur[0], (double)cur[1] * cur[1], (double)cur[2] * cur[2],
+                   (double)cur[3] * cur[3]);
 #pragma unroll
-        for (int u = 0; u < 16; ++u) r[u] = xr[i + u];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) s += (double)r[u] * r[u];
-    }
-    for (; i < width; ++i) {
-        const float v = xr[i];
-        s += (double)v * v;
+        for (int q = 0; q < 4; ++q) cur[q] = nxt[q];
     }
     return s;
 }
@@ -102,7 +137,10 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_kernel(
     }
     __syncthreads();
     if (!ambiguous) return;
-    if (tid == 0) inv_seq = hm_inv_rms(hm_rms_sum_seq(row_lds, width), wd, ed);
+    if (tid < HM_WAVE) {
+        const double s = hm_rms_sum_seq(row_lds, width);
+        if (tid == 0) inv_seq = hm_inv_rms(s, wd, ed);
+    }
     __syncthreads();
     const double inv = inv_seq;
     for (int64_t i = tid; i < width; i += kBlock) {
@@ -115,17 +153,15 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_kernel(
 // together and the row stays in registers (rmsnorm_kernel's strided loop
 // waits for each load before the next).  Same bracket, same fallback (a row
 // with an ambiguous element, or every row with force_seq, takes the
-// sequential sum), with the exact
-// products formed by the whole wave so that lane 0's chain is only the
-// additions.
+// sequential sum, its terms read again from the row: about one row in 128 of
+// N(0, 1) data, and its chain of W additions sets the kernel's time).
 template <int V>
 __global__ __launch_bounds__(kBlock) void rmsnorm_wave_kernel(
     const float* __restrict__ x, const float* __restrict__ gamma,
     float* __restrict__ y, int64_t rows, float eps, int force_seq) {
     constexpr int W = 256 * V;
-    extern __shared__ float row_lds[];  // [4][512] doubles: a chunk of products per wave
-    const int lane = threadIdx.x & (HM_WAVE - 1), wv = threadIdx.x / HM_WAVE;
-    const int64_t r = (int64_t)blockIdx.x * (kBlock / HM_WAVE) + wv;
+    const int lane = threadIdx.x & (HM_WAVE - 1);
+    const int64_t r = (int64_t)blockIdx.x * (kBlock / HM_WAVE) + threadIdx.x / HM_WAVE;
     if (r >= rows) return;
     const float4* xr = reinterpret_cast<const float4*>(x + r * W);
     const float4* g4 = reinterpret_cast<const float4*>(gamma);
@@ -163,53 +199,17 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_wave_kernel(
         one(v[j].w, g.w, out[j].w);
     }
     if (force_seq || __ballot(amb) != 0) {
-        // The reference's sequential sum: s = fl(s + p_k) with the exact
-        // products p_k = double(x_k)^2.  The wave forms the products of 512
-        // consecutive elements (its registers j = 2q, 2q+1) into LDS, then
-        // lane 0 adds them in order, 16 loaded ahead; the chain is one
-        // dependent add per element.
-        double* lp = reinterpret_cast<double*>(row_lds) + (int64_t)wv * 512;
+        const float4* xc = xr + (lane & 15);
         double s = 0.0;
-#pragma unroll
-        for (int q = 0; q < (V + 1) / 2; ++q) {
-            const int nj = 2 * q + 1 < V ? 2 : 1;
-#pragma unroll
-            for (int jj = 0; jj < nj; ++jj) {
-                const float4 x4 = v[2 * q + jj];
-                double* d = lp + 256 * jj + 4 * lane;
-                d[0] = (double)x4.x * x4.x;
-                d[1] = (double)x4.y * x4.y;
-                d[2] = (double)x4.z * x4.z;
-                d[3] = (double)x4.w * x4.w;
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (lane == 0) {
-                const double2* p2 = reinterpret_cast<const double2*>(lp);
-                const int n2 = 128 * nj;  // pairs of products in this chunk
-                double2 cur[8], nxt[8];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) cur[i] = p2[i];
-                for (int b = 0; b < n2; b += 8) {
-                    if (b + 8 < n2) {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) nxt[i] = p2[b + 8 + i];
-                    }
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        s += cur[i].x;
-                        s += cur[i].y;
-                    }
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) cur[i] = nxt[i];
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            __builtin_amdgcn_wave_barrier();
+        float4 cur = xc[0], nxt = xc[16];
+        for (int c = 0; c < W / 64; ++c) {
+            const float4 x4 = cur;
+            cur = nxt;
+            nxt = xc[16 * min(c + 2, W / 64 - 1)];
+            hm_chain64(s, (double)x4.x * x4.x, (double)x4.y * x4.y, (double)x4.z * x4.z,
+                       (double)x4.w * x4.w);
         }
-        double inv = 0.0;
-        if (lane == 0) inv = hm_inv_rms(s, wd, ed);
-        inv = __shfl(inv, 0, HM_WAVE);
+        const double inv = hm_inv_rms(s, wd, ed);
 #pragma unroll
         for (int j = 0; j < V; ++j) {
             const float4 g = g4[HM_WAVE * j + lane];
@@ -227,199 +227,204 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_wave_kernel(
 // A2 router logits (src/router/CpuRouterBackend.cpp:41-49):
 //   logit[t,e] = float(sum_k double(h[t,k]) * double(w[k,e])), k ascending.
 // The product of two floats is exact in double, so fma(h, w, acc) rounds
-// exactly like the reference's multiply-then-add, and each (t, e) chain runs
-// k in order.  Workgroup tile: 16 tokens x 128 experts; thread (tt, te) owns
-// tokens 2tt, 2tt+1 and experts 4te .. 4te+3 (8 independent FMA chains).
-// k is staged through LDS as doubles in 32-wide chunks, double buffered, the
-// next chunk prefetched into registers while the current one is consumed.
+// exactly like the reference's multiply-then-add, and the reference's logit is
+// a chain of fused multiply-adds.  The FP64 matrix instructions compute just
+// that: for every result, v_mfma_f64_16x16x4_f64 and v_mfma_f64_4x4x4_4b_f64
+// add the four products of their k slots to C in ascending order, one fused
+// multiply-add each (verified bit for bit against fma chains: 655,360 results
+// of 256 steps, narrow, wide and full double operands, no difference; the
+// other orders differ in three of four).  So with k slot g of step s holding
+// k = 4 s + g, one accumulator from +0 over all of K is the reference's chain:
+// no bound, no fallback, no workspace.
+//
+// What bounds it: FP64 matrix rate for many tokens (4096 x 2048 x 128: 27 us),
+// and for few the chain itself: 512 dependent 4 x 4 x 4 steps of 21 cycles (5
+// us), the 16 x 16 x 4 form 64 cycles.  One workgroup: 4 waves, 4 C tokens x 64
+// experts, a wave 16 experts; C = 1, 2: one, two 4 x 4 x 4 chains (each of its
+// four blocks the same four tokens and its own four experts), C = 4, 8: one,
+// two 16 x 16 x 4 chains.  W [64 k][64 experts] and h come through a ring of
+// stages in LDS by DMA (16-byte where E % 64 == 0 and w is 16-byte aligned,
+// else 4-byte), one barrier a stage; row k's 16-float groups are stored
+// exchanged by k % 4 and h's rows 68 floats apart, so that the four k slots of
+// a lane group read 64 different banks.  C: a workgroup takes 17, 24, 29 and 46
+// us at H = 2048 (one a CU; a step's conversions and LDS reads, issued by one
+// wave a SIMD, are what lies between these and the chain), so the fewest
+// rounds of workgroups times that.
+//
+// Measured, logits + selection inside a block at H = 2048, E = 128 (before:
+// K ranges summed on the matrix cores, an error bound in the select kernel, and
+// a second sum and chains for what it left open): 61 tokens 16 + 23 -> 21 + 10
+// us, 333 17 + 36 -> 21 + 11 us, 2048 32 + 44 -> 40 + 15 us, 4096 55 + 42 -> 60 +
+// 19 us; 201 tokens of H = 1024, E = 60 (one chain per thread before) 87 + 5 ->
+// 13 + 6 us.
 // ---------------------------------------------------------------------------
-constexpr int kLT = 16;   // tokens per workgroup
-constexpr int kLE = 128;  // experts per workgroup
-constexpr int kLK = 32;   // k per chunk
+constexpr int kCK = 64;   // k per stage
+constexpr int kCH = 68;   // floats from one token's h to the next in a stage
+typedef double hm_double4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(kBlock) void router_logits_kernel(
-    const float* __restrict__ h, const float* __restrict__ w, int64_t tokens,
-    int64_t hidden, int64_t experts, float* __restrict__ logits, int32_t* status) {
-    __shared__ __attribute__((aligned(16))) double hs[2][kLK][kLT];
-    __shared__ __attribute__((aligned(16))) double ws[2][kLK][kLE];
-    const int tid = threadIdx.x;
-    const int tt = tid >> 5, te = tid & 31;
-    const int64_t t0 = (int64_t)blockIdx.x * kLT;
-    const int64_t e0 = (int64_t)blockIdx.y * kLE;
-    // staging: h chunk = 16 x 32 floats (2 per thread), w chunk = 32 x 128
-    // floats (16 per thread, 4 groups of 4 consecutive experts).
-    float hr[2], wr[4][4];
-    auto fetch = [&](int64_t k0) {
+template <int C, bool VEC>
+__global__ __launch_bounds__(256) void router_chain_kernel(
+    const float* __restrict__ h, const float* __restrict__ w, int64_t tokens, int64_t hidden,
+    int experts, float* __restrict__ logits, int32_t* status, int32_t* __restrict__ hist, int hist_n) {
+    constexpr int NI = (VEC ? 4 : 16) + C;  // DMA loads per wave and stage
+    // ring stages: a stage lasts 340 cycles at C = 1 and 2060 at C = 8, a load
+    // from memory about 2000
+    constexpr int kCS = !VEC ? 4 : C == 1 ? 8 : C == 2 ? 6 : 4;
+    static_assert((kCS - 2) * NI <= 63, "vmcnt");
+    constexpr bool BIG = C >= 4;            // 16 x 16 x 4 steps
+    constexpr int NT = BIG ? C / 4 : C;     // chains per wave
+    __shared__ __attribute__((aligned(1024))) float s_w[kCS][kCK][HM_WAVE];
+    __shared__ __attribute__((aligned(1024))) float s_h[kCS][4 * C][kCH];
+    // the permutation's chunk histograms, counted by the select kernel
+    if (blockIdx.y == 0)
+        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < hist_n; i += (int64_t)gridDim.x * 256)
+            hist[i] = 0;
+    const int lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int e0 = blockIdx.y * HM_WAVE;
+    const int64_t t0 = (int64_t)blockIdx.x * (4 * C);
+    const int whole = (int)(hidden / kCK);                  // whole stages
+    const int nm = (int)((hidden + kCK - 1) / kCK);
+    // The next stage's loads (called in stage order): W rows and C of the
+    // tokens' h rows, each from a uniform base, advanced by a stage, and a
+    // 32-bit lane offset; in the last, partial stage rows past the end are the
+    // last row again (the steps there are masked).
+    const int col = VEC ? 4 * (li ^ (4 * g)) : 0;
+    const uint32_t wo = VEC ? (uint32_t)(((4 * wave + g) * experts + e0 + col) * 4) : 0;
+    const float* wb = w;
+    const int64_t wstep = 16 * (int64_t)experts;
+    const float* hb[C];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int idx = tid * 2 + c;
-            const int t = idx / kLK, kk = idx % kLK;
-            const int64_t tg = t0 + t, kg = k0 + kk;
-            hr[c] = (tg < tokens && kg < hidden) ? h[tg * hidden + kg] : 0.0f;
+    for (int n = 0; n < C; ++n) hb[n] = h + min(t0 + C * wave + n, tokens - 1) * hidden;
+    int im = 0, islot = 0;  // the next stage to load and its slot
+    auto issue = [&]() __attribute__((always_inline)) {
+        uint32_t ho = 4u * (uint32_t)lane;
+        if (im < whole) {  // (uniform)
+            if constexpr (VEC) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) dma16_off(wb + q * wstep, wo, &s_w[islot][16 * q + 4 * wave][0]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    dma4_off(wb + (16 * wave + q) * (int64_t)experts,
+                             4u * (uint32_t)min(e0 + (lane ^ (16 * (q & 3))), experts - 1),
+                             &s_w[islot][16 * wave + q][0]);
+            }
+        } else {
+            const int left = (int)(hidden - (int64_t)im * kCK);
+            if constexpr (VEC) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    dma16_off(wb, (uint32_t)((min(16 * q + 4 * wave + g, left - 1) * experts + e0 + col) * 4),
+                              &s_w[islot][16 * q + 4 * wave][0]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 16; ++q)
+                    dma4_off(wb + min(16 * wave + q, left - 1) * (int64_t)experts,
+                             4u * (uint32_t)min(e0 + (lane ^ (16 * (q & 3))), experts - 1),
+                             &s_w[islot][16 * wave + q][0]);
+            }
+            ho = 4u * (uint32_t)min(lane, left - 1);
         }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int idx = tid + kBlock * c;  // 0 .. 1023
-            const int kk = idx >> 5, e4 = idx & 31;
-            const int64_t kg = k0 + kk;
+        for (int n = 0; n < C; ++n) {
+            dma4_off(hb[n], ho, &s_h[islot][C * wave + n][0]);
+            hb[n] += kCK;
+        }
+        wb += 4 * wstep;
+        ++im;
+        islot = islot + 1 == kCS ? 0 : islot + 1;
+    };
+    typedef typename std::conditional<BIG, hm_double4, double>::type Acc;
+    Acc acc[NT];
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
-                const int64_t eg = e0 + 4 * e4 + x;
-                wr[c][x] = (kg < hidden && eg < experts) ? w[kg * experts + eg] : 0.0f;
+    for (int n = 0; n < NT; ++n) acc[n] = Acc{};
+    const int woff = HM_WAVE * g + 16 * (wave ^ g) + li;    // W of k slot g, expert 16 wave + li
+    const int hoff = kCH * (BIG ? li : lane & 3) + g;       // h of k slot g, the lane's token
+    // The operands of four steps (16 k) are a group, group q of a stage in
+    // buffer q, read two groups before its steps: a stage's first two while
+    // the last two of the stage before it run.  So stage m + 1 is waited for
+    // and published half way through stage m, and the slot of stage m - 1,
+    // which every wave has used up by then, takes stage m + kCS - 1.
+    float wv[4][4], hv[4][4][NT];
+    auto read = [&](int slot, auto qc) __attribute__((always_inline)) {
+        constexpr int q = decltype(qc)::value;
+        const float* ws = &s_w[0][0][0] + slot * (kCK * HM_WAVE) + woff;
+        const float* hs = &s_h[0][0][0] + slot * (4 * C * kCH) + hoff;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            wv[q][s] = ws[(16 * q + 4 * s) * HM_WAVE];
+#pragma unroll
+            for (int n = 0; n < NT; ++n) hv[q][s][n] = hs[(BIG ? 16 : 4) * n * kCH + 16 * q + 4 * s];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // (the reads before the steps they overlap)
+    };
+    auto steps = [&](auto qc, auto part, int left) __attribute__((always_inline)) {
+        constexpr int q = decltype(qc)::value;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            // (the last, partial stage: both operands +0 past the end; a chain
+            // from +0 never reaches -0, so adding +0 changes nothing)
+            const bool in = !decltype(part)::value || 16 * q + 4 * s + g < left;
+            const double wd = in ? (double)wv[q][s] : 0.0;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                const double hd = in ? (double)hv[q][s][n] : 0.0;
+                if constexpr (BIG) acc[n] = __builtin_amdgcn_mfma_f64_16x16x4f64(hd, wd, acc[n], 0, 0, 0);
+                else acc[n] = __builtin_amdgcn_mfma_f64_4x4x4f64(hd, wd, acc[n], 0, 0, 0);
             }
         }
     };
-    auto stash = [&](int buf) {
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int idx = tid * 2 + c;
-            hs[buf][idx % kLK][idx / kLK] = (double)hr[c];
+    const std::integral_constant<int, 0> q0;
+    const std::integral_constant<int, 1> q1;
+    const std::integral_constant<int, 2> q2;
+    const std::integral_constant<int, 3> q3;
+    for (int m = 0; m < kCS - 1 && m < nm; ++m) issue();
+    if (nm >= kCS - 1) wait_vmcnt<(kCS - 2) * NI>();
+    else wait_vmcnt<0>();
+    lds_barrier();
+    read(0, q0);
+    read(0, q1);
+    int slot = 0;
+    auto stage = [&](int m, auto part) __attribute__((always_inline)) {
+        const int left = decltype(part)::value ? (int)(hidden - (int64_t)m * kCK) : kCK;
+        read(slot, q2);
+        steps(q0, part, left);
+        read(slot, q3);
+        steps(q1, part, left);
+        const bool more = m + 1 < nm;
+        slot = slot + 1 == kCS ? 0 : slot + 1;
+        if (more) {
+            // stage m + 1 has landed once at most the stages issued after it
+            // are in flight
+            if (m + kCS - 2 < nm) wait_vmcnt<(kCS - 3) * NI>();
+            else wait_vmcnt<0>();
+            lds_barrier();
+            if (im < nm) issue();
+            read(slot, q0);
         }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int idx = tid + kBlock * c;
-            const int kk = idx >> 5, e4 = idx & 31;
-#pragma unroll
-            for (int x = 0; x < 4; ++x) ws[buf][kk][4 * e4 + x] = (double)wr[c][x];
-        }
+        steps(q2, part, left);
+        if (more) read(slot, q1);
+        steps(q3, part, left);
     };
-    double acc[2][4];
+#pragma clang loop unroll(disable)
+    for (int m = 0; m < whole; ++m) stage(m, std::false_type{});
+    if (whole < nm) stage(whole, std::true_type{});
+    // results: 4 x 4 x 4: row lane / 16, column lane % 16 over the four blocks;
+    // 16 x 16 x 4: register r holds row lane / 16 + 4 r, column lane % 16
+    const int e = e0 + 16 * wave + li;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int n = 0; n < NT; ++n) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
-    const int nchunks = (int)((hidden + kLK - 1) / kLK);
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    for (int c = 0; c < nchunks; ++c) {
-        const int buf = c & 1;
-        if (c + 1 < nchunks) fetch((int64_t)(c + 1) * kLK);
-        const int64_t k0 = (int64_t)c * kLK;
-        const int kn = (int)((hidden - k0) < kLK ? (hidden - k0) : kLK);
-        for (int kk = 0; kk < kn; ++kk) {
-            const double h0 = hs[buf][kk][2 * tt], h1 = hs[buf][kk][2 * tt + 1];
-            double wv[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = ws[buf][kk][4 * te + j];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc[0][j] = __builtin_fma(h0, wv[j], acc[0][j]);
-                acc[1][j] = __builtin_fma(h1, wv[j], acc[1][j]);
+        for (int r = 0; r < (BIG ? 4 : 1); ++r) {
+            const int64_t t = t0 + (BIG ? 16 * n + g + 4 * r : 4 * n + g);
+            double v;
+            if constexpr (BIG) v = acc[n][r];
+            else v = acc[n];
+            if (t < tokens && e < experts) {
+                if (!isfinite(v)) hm_status_or(status, HM_STATUS_NONFINITE_SCORE);
+                logits[t * experts + e] = (float)v;
             }
-        }
-        if (c + 1 < nchunks) stash(buf ^ 1);
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int64_t t = t0 + 2 * tt + i;
-        if (t >= tokens) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t e = e0 + 4 * te + j;
-            if (e >= experts) continue;
-            if (!isfinite(acc[i][j])) hm_status_or(status, HM_STATUS_NONFINITE_SCORE);
-            logits[t * experts + e] = (float)acc[i][j];
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// A2 logits, tiled (prefill).  Same arithmetic as router_logits_kernel: one
-// sequential FP64 chain per (token, expert) in ascending k.  Workgroup tile
-// 32 tokens x 64 experts, 256 threads; thread (lt, le) = (tid/16, tid%16)
-// runs the 8 chains of tokens 2lt, 2lt+1 x experts 4le..4le+3, so each k
-// costs three 16-byte LDS reads (two h doubles, four w doubles; the h read
-// is a broadcast across the 16 threads of a token pair) for eight FMAs.
-// W [32 k x 64 e] and h [32 t x 32 k] chunks come straight from global
-// memory into a 4-stage LDS ring (global_load_lds) and are widened to double
-// once per chunk.  Needs E % 64 == 0, H % 32 == 0 and 16-byte aligned h, w.
-// ---------------------------------------------------------------------------
-constexpr int kTT = 32;                // tokens per tile
-constexpr int kTE = 64;                // experts per tile
-constexpr int kTK = 32;                // k per chunk
-constexpr int kTS = 4;                 // ring stages
-constexpr int kTW = kTK * kTE * 4;     // W bytes per stage (8 KB)
-constexpr int kTH = kTT * kTK * 4;     // h bytes per stage (4 KB)
-constexpr int kTLPW = 3;               // 16-byte wave loads per wave per stage
-
-__global__ __launch_bounds__(256) void router_logits_tile_kernel(
-    const float* __restrict__ h, const float* __restrict__ w, int64_t tokens,
-    int64_t hidden, int64_t experts, float* __restrict__ logits, int32_t* status) {
-    __shared__ __attribute__((aligned(1024))) char ring[kTS][kTW + kTH];
-    __shared__ __attribute__((aligned(16))) double hd[kTK][kTT];  // [k][token]
-    __shared__ __attribute__((aligned(16))) double wd[kTK][kTE];  // [k][expert]
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lt = tid >> 4, le = tid & 15;
-    const int64_t t0 = (int64_t)blockIdx.x * kTT;
-    const int64_t e0 = (int64_t)blockIdx.y * kTE;
-    // this wave's loads per stage: W rows [8w, 8w+8) as two 1 KB pieces
-    // (4 rows of 64 floats each), h tokens [8w, 8w+8) x 32 k (8 lanes/token)
-    const float* wsrc0 = w + (8 * wave + (lane >> 4)) * experts + e0 + 4 * (lane & 15);
-    const float* wsrc1 = wsrc0 + 4 * experts;
-    const int64_t tok = min(t0 + 8 * wave + (lane >> 3), tokens - 1);
-    const float* hsrc = h + tok * hidden + 4 * (lane & 7);
-    auto issue = [&](int slot, int64_t k0) {
-        char* st = ring[slot];
-        dma16(wsrc0 + k0 * experts, st + 2048 * wave);
-        dma16(wsrc1 + k0 * experts, st + 2048 * wave + 1024);
-        dma16(hsrc + k0, st + kTW + 1024 * wave);
-    };
-    double acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
-    const int nk = (int)(hidden / kTK);
-#pragma unroll
-    for (int s = 0; s < kTS - 1; ++s)
-        if (s < nk) issue(s, (int64_t)s * kTK);
-    for (int c = 0; c < nk; ++c) {
-        const int slot = c % kTS;
-        if (c + kTS - 2 < nk) wait_vmcnt<(kTS - 2) * kTLPW>();
-        else wait_vmcnt<0>();
-        lds_barrier();  // stage c landed for every wave; chunk c-1 fully computed
-        if (c + kTS - 1 < nk) issue((c + kTS - 1) % kTS, (int64_t)(c + kTS - 1) * kTK);
-        {   // widen the chunk: h thread -> token tid/8, k 4*(tid%8)..+3;
-            // W thread -> floats 4*tid..+3 and 1024+4*tid..+3 of [k][64]
-            const float4 v = *reinterpret_cast<const float4*>(ring[slot] + kTW + 16 * tid);
-            const int t = tid >> 3, kk = 4 * (tid & 7);
-            hd[kk][t] = (double)v.x;
-            hd[kk + 1][t] = (double)v.y;
-            hd[kk + 2][t] = (double)v.z;
-            hd[kk + 3][t] = (double)v.w;
-            const float4 a = *reinterpret_cast<const float4*>(ring[slot] + 16 * tid);
-            const float4 b = *reinterpret_cast<const float4*>(ring[slot] + 4096 + 16 * tid);
-            double* w0 = &wd[0][0] + 4 * tid;
-            w0[0] = (double)a.x; w0[1] = (double)a.y; w0[2] = (double)a.z; w0[3] = (double)a.w;
-            w0[1024] = (double)b.x; w0[1025] = (double)b.y; w0[1026] = (double)b.z; w0[1027] = (double)b.w;
-        }
-        lds_barrier();
-#pragma unroll
-        for (int kk = 0; kk < kTK; ++kk) {
-            const double2 hv = *reinterpret_cast<const double2*>(&hd[kk][2 * lt]);
-            const double2 w01 = *reinterpret_cast<const double2*>(&wd[kk][4 * le]);
-            const double2 w23 = *reinterpret_cast<const double2*>(&wd[kk][4 * le + 2]);
-            acc[0][0] = __builtin_fma(hv.x, w01.x, acc[0][0]);
-            acc[0][1] = __builtin_fma(hv.x, w01.y, acc[0][1]);
-            acc[0][2] = __builtin_fma(hv.x, w23.x, acc[0][2]);
-            acc[0][3] = __builtin_fma(hv.x, w23.y, acc[0][3]);
-            acc[1][0] = __builtin_fma(hv.y, w01.x, acc[1][0]);
-            acc[1][1] = __builtin_fma(hv.y, w01.y, acc[1][1]);
-            acc[1][2] = __builtin_fma(hv.y, w23.x, acc[1][2]);
-            acc[1][3] = __builtin_fma(hv.y, w23.y, acc[1][3]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int64_t t = t0 + 2 * lt + i;
-        if (t >= tokens) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if (!isfinite(acc[i][j])) hm_status_or(status, HM_STATUS_NONFINITE_SCORE);
-            logits[t * experts + e0 + 4 * le + j] = (float)acc[i][j];
         }
     }
 }
@@ -648,41 +653,63 @@ __device__ __forceinline__ float block_logit(const double* __restrict__ pp, int6
 
 // The reference's sequential chain s_k = fl(s_{k-1} + h_k w_k) (the
 // product is exact in double, so fl(s + p) = fma(h, w, s)) for the logit of
-// expert e0 + lane of every lane whose bit is set in `need`, one logit at a time:
-// the whole wave forms 64 exact products at once into LDS (prod: 64
-// doubles of this wave) and the owning lane adds them in order, 16 reads
-// ahead of its additions.  hidden % 16 == 0.  Returns the owning lane's
-// float logit (others: v unchanged).
+// expert e0 + lane of every lane whose bit is set in `need`, four logits at a
+// time, one on each 16-lane row (hm_chain64; the operands D chunks of 64
+// ahead of the chains: a chunk's W column is 64 cache lines, and its chain
+// steps take 250 ns; terms past the end are +0, which leaves every s_k as it
+// is: a chain from +0 never reaches -0).  Returns the owning lane's float
+// logit (others: v unchanged).
+template <int D>
 __device__ __forceinline__ float chain_logits(unsigned long long need, int lane, float v, int64_t e0,
                                               const float* __restrict__ hrow,
                                               const float* __restrict__ w, int64_t hidden,
-                                              int64_t experts, double* prod, int32_t* status) {
+                                              int64_t experts, int32_t* status) {
     while (need) {
-        const int owner = __ffsll((long long)need) - 1;
-        need &= need - 1;
-        const int64_t eo = e0 + owner;
+        // row r takes the r-th needed logit (the last one again past the end)
+        unsigned long long m = need;
+        int owner = 0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = __ffsll((long long)m) - 1;
+            if (r <= (lane >> 4)) owner = o;
+            if (m & (m - 1)) m &= m - 1;
+        }
+        const float* wc = w + e0 + owner;
+        const int64_t i = 4 * (lane & 15);
+        float hv[D][4], wv[D][4];
+        auto load = [&](int64_t k0, int d) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t k = min(k0 + i + q, hidden - 1);
+                hv[d][q] = hrow[k];
+                wv[d][q] = wc[k * experts];
+            }
+        };
+#pragma unroll
+        for (int d = 0; d < D; ++d) load(64 * d, d);
         double acc = 0.0;
-        for (int64_t c0 = 0; c0 < hidden; c0 += HM_WAVE) {
-            const int64_t k = min(c0 + lane, hidden - 1);
-            const double p = (double)hrow[k] * (double)w[k * experts + eo];
-            __builtin_amdgcn_wave_barrier();
-            prod[lane] = p;
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            if (lane == owner) {
-                const int n = (int)min((int64_t)HM_WAVE, hidden - c0);
-                for (int i = 0; i < n; i += 16) {
-                    double r[16];
+        for (int64_t k0 = 0; k0 < hidden; k0 += 64 * D) {
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) r[u] = prod[i + u];
+            for (int d = 0; d < D; ++d) {
+                const int64_t k = k0 + 64 * d;
+                double p[4];
 #pragma unroll
-                    for (int u = 0; u < 16; ++u) acc += r[u];
-                }
+                for (int q = 0; q < 4; ++q)
+                    p[q] = k + i + q < hidden ? (double)hv[d][q] * (double)wv[d][q] : 0.0;
+                load(k + 64 * D, d);
+                hm_chain64(acc, p[0], p[1], p[2], p[3]);
             }
         }
-        if (lane == owner) {
-            if (!isfinite(acc)) hm_status_or(status, HM_STATUS_NONFINITE_SCORE);
-            v = (float)acc;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (!need) break;
+            const int o = __ffsll((long long)need) - 1;
+            need &= need - 1;
+            const double a = __shfl(acc, 16 * r, HM_WAVE);
+            if (lane == o) {
+                if (!isfinite(a)) hm_status_or(status, HM_STATUS_NONFINITE_SCORE);
+                v = (float)a;
+            }
         }
     }
     return v;
@@ -830,7 +857,8 @@ template <int EPL>
 __global__ __launch_bounds__(kBlock) void router_select_kernel(
     const float* __restrict__ logits, int64_t tokens, int64_t experts,
     int32_t top_k, uint32_t flags, uint32_t* __restrict__ ids,
-    float* __restrict__ scores, int32_t* status) {
+    float* __restrict__ scores, int32_t* status, const float* __restrict__ h, int64_t hidden,
+    hm_row_quant xq, int32_t* __restrict__ hist) {
     extern __shared__ float seq_lds[];  // (kBlock/64) * experts floats
     const int lane = threadIdx.x & (HM_WAVE - 1);
     const int wave = threadIdx.x / HM_WAVE;
@@ -846,6 +874,27 @@ __global__ __launch_bounds__(kBlock) void router_select_kernel(
         v[j] = valid[j] ? lt[e] : 0.0f;
     }
     select_token<EPL>(v, valid, lane, wave, t, experts, top_k, flags, ids, scores, status, seq_lds);
+    // The permutation's histogram of each 1024-pair chunk (hm_permute's
+    // count pass): each lane re-reads the id it has just written.  Integer
+    // counts, so the atomics' order does not matter.
+    if (hist && lane < top_k) {
+        const int64_t pr = t * top_k + lane;
+        atomicAdd(&hist[(pr / kPermChunk) * experts + ids[pr]], 1);
+    }
+    // The token's row in fixed-point digits for the INT8 expert GEMMs (the
+    // block's activation quantisation, one launch fewer).
+    if (xq.digits) {
+        const int nv = (int)(hidden / 256);
+        const hm_dlay lay = hm_dlay_x(xq.limbs, hidden);
+        int8_t* d = xq.digits + t * lay.row;
+        int32_t* ds = xq.dsum ? xq.dsum + t : nullptr;
+        const float* hrow = h + t * hidden;
+        switch (xq.limbs) {
+        case 1: hm_quantize_row_wave<1>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
+        case 2: hm_quantize_row_wave<2>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
+        default: hm_quantize_row_wave<3>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
+        }
+    }
 }
 
 // The stable counting sort of permute_count/scatter for at most
@@ -985,7 +1034,6 @@ __global__ __launch_bounds__(NW * HM_WAVE) void router_select_partial_kernel(
     int32_t* __restrict__ offsets, int32_t* __restrict__ perm_tokens,
     float* __restrict__ perm_weights, int32_t* __restrict__ slots, hm_row_quant xq) {
     extern __shared__ float seq_lds[];  // NW * experts floats
-    __shared__ double s_prod[NW][HM_WAVE];
     // one workgroup: the grouping reads the ids and scores from LDS copies
     __shared__ uint32_t s_sel_ids[PERMUTE ? NW * 64 : 1];
     __shared__ float s_sel_sc[PERMUTE ? NW * 64 : 1];
@@ -1011,8 +1059,8 @@ __global__ __launch_bounds__(NW * HM_WAVE) void router_select_partial_kernel(
             v = 0.0f;
             settled = true;
         }
-        v = chain_logits(__ballot(valid && !settled), lane, v, (int64_t)HM_WAVE * j,
-                         h + t * hidden, w, hidden, experts, s_prod[wave], status);
+        v = chain_logits<4>(__ballot(valid && !settled), lane, v, (int64_t)HM_WAVE * j,
+                         h + t * hidden, w, hidden, experts, status);
         if (valid) logits[t * experts + e] = v;
         return v;
     };
@@ -1132,7 +1180,6 @@ __global__ __launch_bounds__(kGvThreads) void select_gateup_kernel(
     extern __shared__ __attribute__((aligned(16))) float s_x[];  // the token row (K32 floats)
     __shared__ double s_b[EPL][kNB][HM_WAVE];
     __shared__ double s_c[EPL][WPR][HM_WAVE];
-    __shared__ double s_prod[EPL][HM_WAVE];
     __shared__ float s_seq[EPL * HM_WAVE];
     __shared__ float s_lg[EPL][HM_WAVE];
     __shared__ uint32_t s_sel_ids[HM_WAVE], s_own_ids[HM_WAVE];
@@ -1187,8 +1234,8 @@ __global__ __launch_bounds__(kGvThreads) void select_gateup_kernel(
         const bool settled = !valid || ((flags & HM_EXEC_ROUTE_SEQUENTIAL) == 0 &&
                                         block_sums_settle(a, sa, sc, hidden));
         float v = valid ? (float)a : 0.0f;
-        v = chain_logits(__ballot(valid && !settled), lane, v, (int64_t)HM_WAVE * wave, h, w,
-                         hidden, experts, s_prod[wave], st);
+        v = chain_logits<1>(__ballot(valid && !settled), lane, v, (int64_t)HM_WAVE * wave, h, w,
+                         hidden, experts, st);
         if (lead && valid) logits[e] = v;
         s_lg[wave][lane] = v;
     }
@@ -1224,481 +1271,6 @@ __global__ __launch_bounds__(kGvThreads) void select_gateup_kernel(
     gateup_slice_body<1, LJ, true, 1>(blockIdx.x, blockIdx.y,
                                       hm_slice_pre{e, (int)blockIdx.y, 1, 0}, h, nullptr, hidden,
                                       inter, experts, packed, scale, zp, nullptr, 1, z);
-}
-
-// ---------------------------------------------------------------------------
-// A2 logits for prefill batches on the FP64 matrix cores, certified.
-//
-// router_mfma_kernel sums the exact products p_k = h_k w_k (double) with
-// v_mfma_f64_16x16x4_f64 in an order of its own: K is cut into `splits`
-// ranges (one per workgroup layer of the grid) and each range into chunks
-// of 16, of which MFMA step j takes k = 4g + j for the four k-slots g; the
-// kernel also returns the norms of h's rows and W's columns per
-// range.  router_select_split_kernel adds the S ranges' partials P'_r in
-// order (S'_r after range r, S' = S'_{S-1}) and bounds |S' - s_n| from
-// these, with m = n / S terms per range, A_r = sum_{k in r} |p_k| <=
-// ||h_r|| ||w_e,r|| (Cauchy-Schwarz per range) and u = 2^-53:
-//   - each range partial: any summation tree of m terms errs by at most
-//     gamma_m A_r, doubled to cover an internal rounding mode of the
-//     matrix cores of up to 2u (g2 = 2mu / (1 - 2mu));
-//   - the additions of the partials: u |S'_r| each; with the above
-//     D = g2 sum_r A_r + u sum_r |S'_r| bounds |S' - S_n| and every prefix
-//     |S'_{r-1} - S_{rm}| (S_k: the exact partial sums);
-//   - the reference's chain: its step k errs by at most u' |s_k| (u' =
-//     u / (1 - u)), |s_k| <= |S_k| + B and, for k in range r, |S_k| <=
-//     |S'_{r-1}| + D + A_r, so B <= u' m (sum_r |S'_{r-1}| + S D + sum_r
-//     A_r) / (1 - n u');
-// the bound is B + D, inflated by 2^-20 for the norms' and the bound's own
-// rounding (relative errors below 2^-40 here).  float(S') is kept when both
-// ends of S' +- bound round to the same float; otherwise (about 0.05 % of
-// the logits for N(0,1) rows and N(0, 0.02) weights at H = 2048 in four
-// ranges, and every non-finite case) the logit takes the fallbacks below.
-//
-// Workgroup: 4 waves x 16 tokens, 64 experts as 4 interleaved MFMA chains
-// (chain q holds experts e0 + 4n + q, n = 0..15), so that each W load is a
-// float4 of 4 consecutive experts (one per chain) and each h load a float4
-// of 4 consecutive k (one per MFMA step).  Lane (g, i) = (lane/16, lane%16)
-// supplies A = h[t0 + i][k] and B = W[k][e0 + 4i + q]; its result register
-// r holds D[g + 4r][i] = the logit of token t0 + g + 4r, expert e0 + 4i + q.
-// Needs E % 64 == 0, H % (16 * splits) == 0, 16-byte aligned h and w.
-// ---------------------------------------------------------------------------
-constexpr int kMT = 64;   // tokens per workgroup
-constexpr int kME = 64;   // experts per workgroup
-constexpr int kMaxSplits = 8;
-constexpr int kMS = 4;    // LDS ring stages of one 16-k chunk each
-constexpr int kMW = 4096; // W bytes per stage: [16 k][64 e] floats
-constexpr int kMH = 4096; // h bytes per stage: [64 t][16 k] floats
-typedef double hm_double4 __attribute__((ext_vector_type(4)));
-
-__global__ __launch_bounds__(256) void router_mfma_kernel(
-    const float* __restrict__ h, const float* __restrict__ w, int tokens, int hidden,
-    int experts, int ksplit, double* __restrict__ part, float* __restrict__ wt,
-    double* __restrict__ hnorm_r, double* __restrict__ wnorm_r, int32_t* __restrict__ hist, int hist_n) {
-    __shared__ __attribute__((aligned(1024))) char ring[kMS][kMW + kMH];
-    // the permutation's chunk histograms, counted by the select kernel
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < hist_n; i += gridDim.x * 256) hist[i] = 0;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = lane >> 4, i = lane & 15;
-    const int eblocks = experts / kME;
-    const int tblocks = (tokens + kMT - 1) / kMT;
-    const int eb = blockIdx.x % eblocks;
-    const int tb = (blockIdx.x / eblocks) % tblocks;
-    const int sp = blockIdx.x / (eblocks * tblocks);
-    const int t0 = tb * kMT + 16 * wave;
-    const int e0 = eb * kME;
-    const int tok = t0 + i;
-    const bool live = tok < tokens;
-    const int kb = sp * ksplit;
-    const int nk = ksplit / 16;
-    // Each wave stages a quarter of a chunk: W rows 4*wave .. +3 (1 KB, lane
-    // l: row 4*wave + l/16, experts 4*(l%16) .. +3) and its own 16 tokens' h
-    // (1 KB, lane l: token 16*wave + l/4, k 4*(l%4) .. +3); rows of tokens
-    // past the end repeat the last token and are masked below.
-    const float* wsrc = w + (int64_t)(kb + 4 * wave + (lane >> 4)) * experts + e0 + 4 * (lane & 15);
-    const int htok = min(t0 + (lane >> 2), tokens - 1);
-    const float* hsrc = h + (int64_t)htok * hidden + kb + 4 * (lane & 3);
-    auto issue = [&](int slot, int c) {
-        dma16(wsrc + (int64_t)16 * c * experts, ring[slot] + 1024 * wave);
-        dma16(hsrc + 16 * c, ring[slot] + kMW + 1024 * wave);
-    };
-    const bool wnorm = tb == 0 && wave == 0;  // one wave per (range, expert block)
-    hm_double4 acc[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) acc[q] = hm_double4{0.0, 0.0, 0.0, 0.0};
-    double hsq = 0.0, wsq[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int c = 0; c < kMS - 1; ++c)
-        if (c < nk) issue(c, c);
-    // The K loop, in four copies: with or without h's squares (the waves of
-    // expert block 0 write them) and W's squares (wnorm); the choice is made
-    // once per wave, outside the loop (every copy takes the same barriers).
-    auto kloop = [&](auto hs, auto ws) __attribute__((always_inline)) {
-        constexpr bool HS = decltype(hs)::value, WS = decltype(ws)::value;
-        for (int c = 0; c < nk; ++c) {
-            const int slot = c % kMS;
-            if (c + kMS - 2 < nk) wait_vmcnt<(kMS - 2) * 2>();
-            else wait_vmcnt<0>();
-            lds_barrier();  // chunk c landed for every wave; chunk c-1 fully read
-            if (c + kMS - 1 < nk) issue((c + kMS - 1) % kMS, c + kMS - 1);
-            const char* st = ring[slot];
-            if (tb == 0) {
-                // the first token block also writes the chunk of W transposed:
-                // lane l -> expert e0 + 16*wave + l/4, k 4*(l%4) .. +3
-                const int ex = 16 * wave + (lane >> 2), kq = 4 * (lane & 3);
-                const float* sw = reinterpret_cast<const float*>(st) + kq * kME + ex;
-                *reinterpret_cast<float4*>(wt + (int64_t)(e0 + ex) * hidden + kb + 16 * c + kq) =
-                    make_float4(sw[0], sw[kME], sw[2 * kME], sw[3 * kME]);
-            }
-            const float4 a = *reinterpret_cast<const float4*>(st + kMW + (16 * wave + i) * 64 + 16 * g);
-            float4 wv[4];
-    #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                wv[j] = *reinterpret_cast<const float4*>(st + (4 * g + j) * 256 + 16 * i);
-            const double ad[4] = {live ? (double)a.x : 0.0, live ? (double)a.y : 0.0,
-                                  live ? (double)a.z : 0.0, live ? (double)a.w : 0.0};
-    #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if constexpr (HS) hsq = __builtin_fma(ad[j], ad[j], hsq);
-                const double bd[4] = {(double)wv[j].x, (double)wv[j].y, (double)wv[j].z,
-                                      (double)wv[j].w};
-    #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(ad[j], bd[q], acc[q], 0, 0, 0);
-                if constexpr (WS) {
-    #pragma unroll
-                    for (int q = 0; q < 4; ++q) wsq[q] = __builtin_fma(bd[q], bd[q], wsq[q]);
-                }
-            }
-        }
-    };
-    if (eb == 0) {
-        if (wnorm) kloop(std::true_type{}, std::true_type{});
-        else kloop(std::true_type{}, std::false_type{});
-    } else {
-        if (wnorm) kloop(std::false_type{}, std::true_type{});
-        else kloop(std::false_type{}, std::false_type{});
-    }
-    // partial logits: register r of lane (g, i) holds D[g + 4r][i], i.e.
-    // token t0 + g + 4r, experts e0 + 4i .. +3
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int t = t0 + g + 4 * r;
-        if (t < tokens) {
-            double* o = part + ((int64_t)sp * tokens + t) * experts + e0 + 4 * i;
-            *reinterpret_cast<double2*>(o) = double2{acc[0][r], acc[1][r]};
-            *reinterpret_cast<double2*>(o + 2) = double2{acc[2][r], acc[3][r]};
-        }
-    }
-    // norms over this range: the four k-slots of a token / expert are the
-    // lanes i, i + 16, i + 32, i + 48
-    hsq += __shfl_xor(hsq, 16, HM_WAVE);
-    hsq += __shfl_xor(hsq, 32, HM_WAVE);
-    // (the norms themselves: their square roots, once here rather than for
-    // every logit in the select kernel)
-    if (eb == 0 && g == 0 && live) hnorm_r[(int64_t)sp * tokens + tok] = sqrt(hsq);
-    if (wnorm) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            wsq[q] += __shfl_xor(wsq[q], 16, HM_WAVE);
-            wsq[q] += __shfl_xor(wsq[q], 32, HM_WAVE);
-        }
-        if (g == 0) {
-            double* o = wnorm_r + (int64_t)sp * experts + e0 + 4 * i;
-            *reinterpret_cast<double2*>(o) = double2{sqrt(wsq[0]), sqrt(wsq[1])};
-            *reinterpret_cast<double2*>(o + 2) = double2{sqrt(wsq[2]), sqrt(wsq[3])};
-        }
-    }
-}
-
-// Fallback chains of the split select.  A wave's uncertified logits are
-// taken kFN at a time: lane f < kFN runs the reference's chain (k
-// ascending) for the f-th of them.  The whole wave stages the next
-// kFK-long piece of their W columns (rows of the transposed copy the
-// matrix-core kernel wrote) and of the token's h row into LDS with 16-byte
-// DMA (double-buffered), then forms that piece's exact products
-// double(h_k) * double(w_k) (48-bit, exact in FP64) for both chains in an
-// LDS product buffer, so a chain step is one dependent FP64 add,
-// acc + p_k == fma(h_k, w_k, acc), with no conversions on its path.
-constexpr int kFK = 128;                        // k per staged piece
-constexpr int kFN = 2;                          // chains per round
-constexpr int kFS = 3;                          // pieces in the staging ring (LDS: four
-                                                // workgroups per CU)
-constexpr int kFBuf = 4 * kFK * 4;              // one buffer: 2 columns, h, pad (2 KB)
-constexpr int kFProd = kFN * kFK * 8;           // products of one piece (2 KB)
-constexpr int kFWave = kFS * kFBuf + kFProd;    // fallback LDS per wave
-constexpr int kFDma = 2;                        // 16-byte DMA instructions per piece
-static_assert(kFK == 2 * HM_WAVE && kFN == 2, "half a wave per staged row piece");
-static_assert(kFS == 3, "the staging waits below count three pieces");
-
-__device__ __forceinline__ void fallback_issue(char* buf, const float* __restrict__ hrow,
-                                               const float* __restrict__ wt, int64_t hidden,
-                                               int64_t k0, const int (&fe)[kFN], int lane) {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this buffer's last reads are done
-    const int half = lane >> 5;
-    const int64_t k = min(k0 + 4 * (lane & 31), hidden - 4);  // past the end: unused
-    // lanes 0-31: column 0, lanes 32-63: column 1; then h twice (the second
-    // copy lands in the pad)
-    dma16(wt + (int64_t)fe[half] * hidden + k, buf);
-    dma16(hrow + k, buf + 2 * 4 * kFK);
-}
-
-// The idx-th set bit over the masks need[0..EPL) in (j, lane) order:
-// its lane and j.
-template <int EPL>
-__device__ __forceinline__ void locate_fallback(const unsigned long long (&need)[EPL], int idx,
-                                                int& owner, int& slot) {
-    int jj = 0;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-        const int c = __popcll(need[j]);
-        if (jj == j && idx >= c) { idx -= c; jj = j + 1; }
-    }
-    unsigned long long m = need[0];
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) if (j == jj) m = need[j];
-    for (int b = 0; b < idx; ++b) m &= m - 1;
-    owner = __ffsll((long long)m) - 1;
-    slot = jj;
-}
-
-template <int EPL>
-__global__ __launch_bounds__(kBlock) void router_select_split_kernel(
-    const float* __restrict__ h, const float* __restrict__ wt, const double* __restrict__ part,
-    const double* __restrict__ hnorm_r, const double* __restrict__ wnorm_r, int64_t tokens,
-    int64_t hidden, int64_t experts, int splits, int32_t top_k, uint32_t flags,
-    float* __restrict__ logits, uint32_t* __restrict__ ids, float* __restrict__ scores,
-    int32_t* status, hm_row_quant xq, int32_t* __restrict__ hist) {
-    // per wave: experts floats for the sequential softmax sum, then the
-    // fallback chains' staging ring and products (kFWave, 16-byte aligned)
-    extern __shared__ __attribute__((aligned(16))) char dyn_lds[];
-    const int lane = threadIdx.x & (HM_WAVE - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / HM_WAVE);
-    const int64_t t = (int64_t)blockIdx.x * (kBlock / HM_WAVE) + wave;
-    if (t >= tokens) return;
-    const int64_t seq_stride = ((experts * 4 + 15) / 16) * 16;
-    float* seq_lds = reinterpret_cast<float*>(dyn_lds);  // indexed by wave * experts
-    char* fb = dyn_lds + (kBlock / HM_WAVE) * seq_stride + (int64_t)wave * kFWave;
-    double* fprod = reinterpret_cast<double*>(fb + kFS * kFBuf);
-    const double u = 0x1p-53;
-    const double n = (double)hidden, m = (double)(hidden / splits);
-    // the range form's bound (derived above router_mfma_kernel)
-    const double g2 = 2.0 * m * u / (1.0 - 2.0 * m * u);
-    const double cu = u / (1.0 - u) / (1.0 - n * u / (1.0 - u)) * m;
-    // (all loads of the range sums go out before the additions:
-    // unconditional loads from clamped ranges, so that no branch splits
-    // them from their uses)
-    double hr[kMaxSplits];
-#pragma unroll
-    for (int sp = 0; sp < kMaxSplits; ++sp)
-        hr[sp] = hnorm_r[(int64_t)min(sp, splits - 1) * tokens + t];
-    float v[EPL];
-    bool valid[EPL];
-    unsigned long long need[EPL];
-    int total = 0;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-        const int64_t e = lane + (int64_t)HM_WAVE * j;
-        valid[j] = e < experts;
-        bool nd = false;
-        v[j] = 0.0f;
-        if (valid[j]) {
-            double pa[kMaxSplits], pw[kMaxSplits];
-#pragma unroll
-            for (int sp = 0; sp < kMaxSplits; ++sp) {
-                const int64_t sc = min(sp, splits - 1);
-                pa[sp] = part[(sc * tokens + t) * experts + e];
-                pw[sp] = wnorm_r[sc * experts + e];
-            }
-            // S' (the ranges' partials added in order), the sums of |S'|
-            // before (pre) and after (post) each addition, and of the
-            // ranges' norm products
-            double a = 0.0, pre = 0.0, post = 0.0, nsum = 0.0;
-#pragma unroll
-            for (int sp = 0; sp < kMaxSplits; ++sp) {
-                if (sp < splits) {
-                    pre += fabs(a);
-                    a += pa[sp];
-                    post += fabs(a);
-                    nsum += hr[sp] * pw[sp];
-                }
-            }
-            // nsum bounds sum_r sum_{k in r} |p_k| (Cauchy-Schwarz per range;
-            // the computed norms err by at most gamma_m relative, covered by
-            // the final inflation)
-            const double d = g2 * nsum + u * post;
-            const double bc = (cu * (pre + (double)splits * d + nsum) + d) * (1.0 + 0x1p-20);
-            const double lo = a - bc, hi = a + bc;
-            nd = !(isfinite(lo) && isfinite(hi) &&
-                   __float_as_uint((float)lo) == __float_as_uint((float)hi));
-            v[j] = (float)a;
-        }
-        need[j] = __ballot(nd);
-        total += __popcll(need[j]);
-    }
-    const float* hrow = h + t * hidden;
-    if (total > 0 && hidden % (kNB * 16) == 0) {
-        // Second level: the decode path's block form and its much tighter
-        // bound, two logits at a time, lane 32*half + j summing block j of
-        // the half's logit (b = H/32 terms, sequentially from +0) beside
-        // R_j and Q_j; the block sums are then chained in order.  Logits it
-        // settles leave the list; the rest take the full chain below.
-        const int half = lane >> 5, bj = lane & 31;
-        const int64_t bw = hidden / kNB;
-        bool left[EPL];
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) left[j] = (need[j] >> lane) & 1ull;
-        for (int done = 0; done < total; done += 2) {  // wave-uniform
-            const int idx = min(done + half, total - 1);
-            int owner, js;
-            locate_fallback<EPL>(need, idx, owner, js);
-            const int64_t e = owner + (int64_t)HM_WAVE * js;
-            const float* hp = hrow + bj * bw;
-            const float* wp = wt + e * hidden + bj * bw;
-            double acc = 0.0, rs = 0.0, qs = 0.0;
-            // 16 k per step; the next step's loads go out before this step's
-            // chains (the last step loads its own chunk again)
-            float4 hv[4], wv[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                hv[q] = *reinterpret_cast<const float4*>(hp + 4 * q);
-                wv[q] = *reinterpret_cast<const float4*>(wp + 4 * q);
-            }
-            for (int64_t k0 = 0; k0 < bw; k0 += 16) {
-                const int64_t kn = k0 + 16 < bw ? k0 + 16 : k0;
-                float4 hn[4], wn[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    hn[q] = *reinterpret_cast<const float4*>(hp + kn + 4 * q);
-                    wn[q] = *reinterpret_cast<const float4*>(wp + kn + 4 * q);
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float hq[4] = {hv[q].x, hv[q].y, hv[q].z, hv[q].w};
-                    const float wq[4] = {wv[q].x, wv[q].y, wv[q].z, wv[q].w};
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const double hk = (double)hq[r], wk = (double)wq[r];
-                        acc = __builtin_fma(hk, wk, acc);  // == acc + hk * wk
-                        rs += fabs(acc);
-                        qs = __builtin_fma(fabs(hk), fabs(wk), qs);
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) { hv[q] = hn[q]; wv[q] = wn[q]; }
-            }
-            const double cj = block_c_term(rs, qs, hidden);
-            double a = 0.0, sa = 0.0, sc = 0.0;
-#pragma unroll
-            for (int j = 0; j < kNB; ++j) {
-                a += __shfl(acc, 32 * half + j, HM_WAVE);
-                sa += fabs(a);
-                sc += __shfl(cj, 32 * half + j, HM_WAVE);
-            }
-            const bool ok = block_sums_settle(a, sa, sc, hidden);
-            // the owners of this pass's logits take the settled values
-#pragma unroll
-            for (int hf = 0; hf < 2; ++hf) {
-                const int o = __shfl(owner, 32 * hf, HM_WAVE);
-                const int jo = __shfl(js, 32 * hf, HM_WAVE);
-                const bool okh = __shfl((int)ok, 32 * hf, HM_WAVE) != 0;
-                const float vh = __shfl((float)a, 32 * hf, HM_WAVE);
-                if (okh && lane == o && (hf == 0 || done + 1 < total)) {
-#pragma unroll
-                    for (int j = 0; j < EPL; ++j) if (j == jo) { v[j] = vh; left[j] = false; }
-                }
-            }
-        }
-        total = 0;
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) {
-            need[j] = __ballot(left[j]);
-            total += __popcll(need[j]);
-        }
-    }
-    for (int done = 0; done < total; done += kFN) {  // wave-uniform
-        // the experts of fallbacks done .. done + kFN - 1 (in (j, lane)
-        // order; slots past the last repeat it)
-        int fe[kFN];
-        int owner[kFN], slot[kFN];
-#pragma unroll
-        for (int f = 0; f < kFN; ++f) {
-            locate_fallback<EPL>(need, min(done + f, total - 1), owner[f], slot[f]);
-            fe[f] = owner[f] + HM_WAVE * slot[f];
-        }
-        const int nf = min(kFN, total - done);
-        double acc = 0.0;
-        const int64_t pieces = (hidden + kFK - 1) / kFK;
-#pragma unroll
-        for (int c = 0; c < kFS - 1; ++c)
-            if (c < pieces) fallback_issue(fb + c * kFBuf, hrow, wt, hidden, c * kFK, fe, lane);
-        for (int64_t c = 0; c < pieces; ++c) {
-            char* cur = fb + (c % kFS) * kFBuf;
-            // the piece kFS - 1 ahead goes into the buffer piece c - 1 used
-            // (fallback_issue waits for its reads)
-            if (c + kFS - 1 < pieces)
-                fallback_issue(fb + ((c + kFS - 1) % kFS) * kFBuf, hrow, wt, hidden,
-                               (c + kFS - 1) * kFK, fe, lane);
-            // piece c has landed once at most the pieces issued after it are
-            // in flight (each piece is kFDma loads; nothing else is loaded here)
-            const int64_t after = min((int64_t)kFS - 1, pieces - 1 - c);
-            if (after >= 2) wait_vmcnt<2 * kFDma>();
-            else if (after == 1) wait_vmcnt<kFDma>();
-            else wait_vmcnt<0>();
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            const int kc = (int)min((int64_t)kFK, hidden - c * kFK);  // a multiple of 16
-            {
-                // the piece's products: lane l forms k = 2l, 2l+1 of both chains
-                const float2 hv = reinterpret_cast<const float2*>(cur + 2 * 4 * kFK)[lane];
-                const float2 w0 = reinterpret_cast<const float2*>(cur)[lane];
-                const float2 w1 = reinterpret_cast<const float2*>(cur + 4 * kFK)[lane];
-                const double h0 = (double)hv.x, h1 = (double)hv.y;
-                reinterpret_cast<double2*>(fprod)[lane] = double2{h0 * (double)w0.x, h1 * (double)w0.y};
-                reinterpret_cast<double2*>(fprod + kFK)[lane] = double2{h0 * (double)w1.x, h1 * (double)w1.y};
-            }
-            // (one wave's LDS accesses complete in order: the chain lanes'
-            // reads below see every lane's products)
-            if (lane < nf) {
-                // 16 products per step, the next step's read out while this
-                // one's are added (kc is a multiple of 16)
-                const double2* pp = reinterpret_cast<const double2*>(fprod + lane * kFK);
-                double2 pa[8];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) pa[q] = pp[q];
-                for (int kk = 0; kk < kc; kk += 16) {
-                    const int nx = kk + 16 < kc ? (kk + 16) / 2 : kk / 2;
-                    double2 pb[8];
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) pb[q] = pp[nx + q];
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) {
-                        acc = acc + pa[q].x;
-                        acc = acc + pa[q].y;
-                    }
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) pa[q] = pb[q];
-                }
-            }
-            // the products are rewritten for the next piece only after
-            // the chains have read them
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        }
-        if (lane < nf && !isfinite(acc)) hm_status_or(status, HM_STATUS_NONFINITE_SCORE);
-#pragma unroll
-        for (int f = 0; f < kFN; ++f) {
-            const double r = __shfl(acc, f, HM_WAVE);
-            if (f < nf && lane == owner[f]) {
-#pragma unroll
-                for (int j = 0; j < EPL; ++j) if (j == slot[f]) v[j] = (float)r;
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < EPL; ++j)
-        if (valid[j] && logits) logits[t * experts + lane + HM_WAVE * j] = v[j];
-    select_token<EPL>(v, valid, lane, wave, t, experts, top_k, flags, ids, scores, status,
-                      seq_lds);
-    // The permutation's histogram of each 1024-pair chunk (hm_permute's
-    // count pass): each lane re-reads the id it has just written.  Integer
-    // counts, so the atomics' order does not matter.
-    if (hist && lane < top_k) {
-        const int64_t pr = t * top_k + lane;
-        atomicAdd(&hist[(pr / kPermChunk) * experts + ids[pr]], 1);
-    }
-    // The token's row in fixed-point digits for the INT8 expert GEMMs (the
-    // block's activation quantisation, fused here: this kernel's time is set
-    // by a few waves' sequential chains, the rest of the machine is idle).
-    if (xq.digits) {
-        const int nv = (int)(hidden / 256);
-        const hm_dlay lay = hm_dlay_x(xq.limbs, hidden);
-        int8_t* d = xq.digits + t * lay.row;
-        int32_t* ds = xq.dsum ? xq.dsum + t : nullptr;
-        switch (xq.limbs) {
-        case 1: hm_quantize_row_wave<1>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
-        case 2: hm_quantize_row_wave<2>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
-        default: hm_quantize_row_wave<3>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
-        }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1963,12 +1535,11 @@ int hm_launch_rmsnorm(const float* x, const float* gamma, float* y, int64_t rows
     const bool aligned = ((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)y) % 16 == 0;
     if (aligned && width % 256 == 0 && width / 256 <= 16) {
         const unsigned grid = (unsigned)((rows + kBlock / HM_WAVE - 1) / (kBlock / HM_WAVE));
-        const size_t lds = (size_t)(kBlock / HM_WAVE) * 512 * sizeof(double);
         const hipStream_t s = hm_stream(stream);
         const int fs = force_seq ? 1 : 0;
         switch (width / 256) {
 #define HM_RMS_CASE(v) \
-    case v: hipLaunchKernelGGL(rmsnorm_wave_kernel<v>, dim3(grid), dim3(kBlock), lds, s, x, gamma, y, rows, eps, fs); break;
+    case v: hipLaunchKernelGGL(rmsnorm_wave_kernel<v>, dim3(grid), dim3(kBlock), 0, s, x, gamma, y, rows, eps, fs); break;
             HM_RMS_CASE(1) HM_RMS_CASE(2) HM_RMS_CASE(3) HM_RMS_CASE(4) HM_RMS_CASE(5) HM_RMS_CASE(6)
             HM_RMS_CASE(7) HM_RMS_CASE(8) HM_RMS_CASE(9) HM_RMS_CASE(10) HM_RMS_CASE(11)
             HM_RMS_CASE(12) HM_RMS_CASE(13) HM_RMS_CASE(14) HM_RMS_CASE(15) HM_RMS_CASE(16)
@@ -1992,45 +1563,63 @@ int hm_rmsnorm(const float* x, const float* gamma, float* y, int64_t rows,
 }
 
 
-// Route workspace: the logits [T x E] floats (rounded up to 256 bytes),
-// then for decode batches (T <= kDecodeTokens) the block partials
-// [T x E x 2 x kNB] doubles, and for prefill batches with E % 64 == 0 the
-// matrix-core range partials [S x T x E] doubles, W transposed [E x H]
-// floats, row norms [S x T] and column norms [S x E] doubles
-// (S = prefill_splits).
+// Route workspace: the logits [T x E] floats (rounded up to 256 bytes), then
+// for decode batches (T <= kDecodeTokens) the block partials
+// [T x E x 2 x kNB] doubles.
 constexpr int64_t kDecodeTokens = 16;
 
 static size_t route_logits_bytes(int64_t tokens, int64_t experts) {
     return ((size_t)tokens * (size_t)experts * sizeof(float) + 255) & ~(size_t)255;
 }
 
-// K ranges of the prefill logits: enough workgroups (>= 512) to give every
-// SIMD two waves; H must also be a multiple of 16 per range (the launcher
-// halves S until it is).
-static int prefill_splits(int64_t tokens, int64_t experts) {
-    const int64_t base = ((tokens + kMT - 1) / kMT) * (experts / kME);
-    int sp = 1;
-    while (sp < kMaxSplits && base * sp < 512) sp *= 2;
-    return sp;
-}
-
 size_t hm_route_workspace_bytes(int64_t tokens, int64_t hidden, int64_t experts) {
     if (tokens < 0 || experts <= 0 || hidden <= 0) return 0;
-    if (tokens > kDecodeTokens) {
-        size_t b = route_logits_bytes(tokens, experts);
-        if (experts % kME == 0) {
-            const size_t sp = (size_t)prefill_splits(tokens, experts);
-            b += sp * ((size_t)tokens * (size_t)experts + (size_t)tokens + (size_t)experts) *
-                     sizeof(double) +
-                 (size_t)experts * (size_t)hidden * sizeof(float);
-        }
-        return b;
-    }
+    if (tokens > kDecodeTokens) return route_logits_bytes(tokens, experts);
     return route_logits_bytes(tokens, experts) +
            (size_t)tokens * (size_t)experts * kNB * 2 * sizeof(double);
 }
 
 }  // extern "C"
+
+// The logits of a batch (router_chain_kernel); hc: the permutation's chunk
+// histograms to clear.
+static int launch_router_chains(const float* h, const float* w, int64_t tokens, int64_t hidden,
+                                int64_t experts, float* logits, int32_t* status, int32_t* hc,
+                                int hc_n, void* stream) {
+    const int64_t eb = (experts + HM_WAVE - 1) / HM_WAVE;
+    // 4 C tokens a workgroup: the shortest rounds of workgroups (above
+    // router_chain_kernel)
+    const int chains[4] = {1, 2, 4, 8};
+    const double cost[4] = {17.0, 24.0, 29.0, 46.0};
+    int c = 1;
+    double best = 0.0;
+    for (int i = 0; i < 4; ++i) {
+        const int64_t wgs = (tokens + 4 * chains[i] - 1) / (4 * chains[i]) * eb;
+        const double us = (double)((wgs + 255) / 256) * cost[i];
+        if (i == 0 || us < best) {
+            best = us;
+            c = chains[i];
+        }
+    }
+    const dim3 grid((unsigned)((tokens + 4 * c - 1) / (4 * c)), (unsigned)eb);
+    const bool vec = experts % HM_WAVE == 0 && (uintptr_t)w % 16 == 0;
+#define HM_CHAINS(C)                                                                            \
+    do {                                                                                        \
+        if (vec)                                                                                \
+            hipLaunchKernelGGL((router_chain_kernel<C, true>), grid, dim3(256), 0, hm_stream(stream), \
+                               h, w, tokens, hidden, (int)experts, logits, status, hc, hc_n);   \
+        else                                                                                    \
+            hipLaunchKernelGGL((router_chain_kernel<C, false>), grid, dim3(256), 0, hm_stream(stream), \
+                               h, w, tokens, hidden, (int)experts, logits, status, hc, hc_n);   \
+    } while (0)
+    if (c == 1) HM_CHAINS(1);
+    else if (c == 2) HM_CHAINS(2);
+    else if (c == 4) HM_CHAINS(4);
+    else HM_CHAINS(8);
+#undef HM_CHAINS
+    HM_LAUNCHED();
+    return HM_OK;
+}
 
 // The decode router's two launches.  With `fused`, the select kernel also
 // forms the expert groups (the workgroup that finishes last) and the
@@ -2214,7 +1803,7 @@ int hm_router_topk(const float* h, const float* w, int64_t tokens,
                                 nullptr, stream);
 }
 
-// hm_router_topk, and where the prefill select kernel runs, the rows of h
+// hm_router_topk, and where a batch's select kernel runs, the rows of h
 // quantised into xq's digit planes as well (*quantized tells the caller).
 __attribute__((visibility("hidden"))) int hm_router_topk_quant(const float* h, const float* w, int64_t tokens,
                          int64_t hidden, int64_t experts, int32_t top_k,
@@ -2229,7 +1818,7 @@ __attribute__((visibility("hidden"))) int hm_router_topk_quant(const float* h, c
     HM_REQUIRE(h && w && ids && scores && tokens > 0 && hidden > 0);
     HM_REQUIRE(logits_out || route_ws);
     if (experts > 1024 || top_k > kMaxTopK) return HM_ERR_UNSUPPORTED;
-    if (tokens > ((int64_t)1 << 31) / kLT) return HM_ERR_OVERFLOW;
+    if (tokens > (int64_t)1 << 27) return HM_ERR_OVERFLOW;  // 32-bit grids
     float* logits = logits_out ? logits_out : static_cast<float*>(route_ws);
     const int epl = (int)((experts + HM_WAVE - 1) / HM_WAVE);
     const dim3 sgrid((unsigned)((tokens + 3) / 4));
@@ -2240,65 +1829,22 @@ __attribute__((visibility("hidden"))) int hm_router_topk_quant(const float* h, c
         return launch_decode_router(h, w, tokens, hidden, experts, top_k, flags, logits, ids,
                                     scores, status, route_ws, nullptr, nullptr, nullptr, stream);
     }
-    const bool aligned = ((uintptr_t)h % 16 == 0) && ((uintptr_t)w % 16 == 0);
-    if (route_ws && !(flags & HM_EXEC_ROUTE_SEQUENTIAL) && aligned && experts % kME == 0 &&
-        hidden % 16 == 0 && hidden <= INT_MAX && tokens <= INT_MAX &&
-        (uintptr_t)route_ws % 16 == 0) {
-        // prefill: matrix-core range partials, then certify + select
-        int sp = prefill_splits(tokens, experts);
-        while (sp > 1 && hidden % (16 * sp) != 0) sp /= 2;
-        double* part = reinterpret_cast<double*>(static_cast<char*>(route_ws) +
-                                                 route_logits_bytes(tokens, experts));
-        float* wt = reinterpret_cast<float*>(part + (int64_t)sp * tokens * experts);
-        double* hnorm_r = reinterpret_cast<double*>(wt + experts * hidden);
-        double* wnorm_r = hnorm_r + (int64_t)sp * tokens;
-        const int64_t grid = ((tokens + kMT - 1) / kMT) * (experts / kME) * sp;
-        // the chunk histograms of hm_permute, when the caller passes them
-        const int64_t chunks = (tokens * top_k + kPermChunk - 1) / kPermChunk;
-        int32_t* hc = hist && chunks > 1 && chunks * experts <= INT_MAX ? hist : nullptr;
-        if (hc && counted) *counted = true;
-        hipLaunchKernelGGL(router_mfma_kernel, dim3((unsigned)grid), dim3(256), 0,
-                           hm_stream(stream), h, w, (int)tokens, (int)hidden, (int)experts,
-                           (int)(hidden / sp), part, wt, hnorm_r, wnorm_r, hc,
-                           hc ? (int)(chunks * experts) : 0);
-        HM_LAUNCHED();
-        const size_t split_bytes =
-            (kBlock / HM_WAVE) * ((((size_t)experts * 4 + 15) / 16) * 16 + (size_t)kFWave);
-        hm_row_quant q = {nullptr, nullptr, nullptr, 0};
-        if (xq && xq->digits && xq->scales && xq->limbs >= 1 && xq->limbs <= 3 &&
-            hidden % 256 == 0 && hidden / 256 <= kHmQuantMaxV &&
-            (uintptr_t)xq->digits % 4 == 0) {
-            q = *xq;
-            if (quantized) *quantized = true;
-        }
-#define HM_SELECTS(N)                                                                     \
-        hipLaunchKernelGGL(router_select_split_kernel<N>, sgrid, dim3(kBlock), split_bytes, \
-                           hm_stream(stream), h, wt, part, hnorm_r, wnorm_r, tokens, hidden, experts, \
-                           sp, top_k, flags, logits, ids, scores, status, q, hc)
-        if (epl <= 1) HM_SELECTS(1);
-        else if (epl <= 2) HM_SELECTS(2);
-        else if (epl <= 4) HM_SELECTS(4);
-        else if (epl <= 8) HM_SELECTS(8);
-        else HM_SELECTS(16);
-#undef HM_SELECTS
-        HM_LAUNCHED();
-        return HM_OK;
-    }
-    if (aligned && experts % kTE == 0 && hidden % kTK == 0) {
-        const dim3 grid((unsigned)((tokens + kTT - 1) / kTT), (unsigned)(experts / kTE));
-        hipLaunchKernelGGL(router_logits_tile_kernel, grid, dim3(256), 0, hm_stream(stream), h,
-                           w, tokens, hidden, experts, logits, status);
-    } else {
-        const dim3 lgrid((unsigned)((tokens + kLT - 1) / kLT),
-                         (unsigned)((experts + kLE - 1) / kLE));
-        hipLaunchKernelGGL(router_logits_kernel, lgrid, dim3(kBlock), 0, hm_stream(stream),
-                           h, w, tokens, hidden, experts, logits, status);
-    }
-    HM_LAUNCHED();
+    hm_row_quant bq = {nullptr, nullptr, nullptr, 0};
+    if (xq && xq->digits && xq->scales && xq->limbs >= 1 && xq->limbs <= 3 && hidden % 256 == 0 &&
+        hidden / 256 <= kHmQuantMaxV && (uintptr_t)xq->digits % 4 == 0 && (uintptr_t)h % 16 == 0)
+        bq = *xq;
+    // the chunk histograms of hm_permute, when the caller passes them
+    const int64_t chunks = (tokens * top_k + kPermChunk - 1) / kPermChunk;
+    int32_t* hc = hist && chunks > 1 && chunks * experts <= INT_MAX ? hist : nullptr;
+    const int hc_n = hc ? (int)(chunks * experts) : 0;
+    if (quantized) *quantized = bq.digits != nullptr;
+    if (counted) *counted = hc != nullptr;
+    const int rc = launch_router_chains(h, w, tokens, hidden, experts, logits, status, hc, hc_n, stream);
+    if (rc) return rc;
 #define HM_SELECT(N)                                                                   \
     hipLaunchKernelGGL(router_select_kernel<N>, sgrid, dim3(kBlock), seq_bytes,        \
                        hm_stream(stream), logits, tokens, experts, top_k, flags, ids,  \
-                       scores, status)
+                       scores, status, h, hidden, bq, hc)
     if (epl <= 1) HM_SELECT(1);
     else if (epl <= 2) HM_SELECT(2);
     else if (epl <= 4) HM_SELECT(4);

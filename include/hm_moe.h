@@ -129,12 +129,11 @@ int hm_rmsnorm(const float* x, const float* gamma, float* y, int64_t rows,
  * the selected scores in rank order.  ids/scores are [tokens x top_k] in
  * rank order.  Bit-exact.  The logits go to logits_out, or, when it is NULL,
  * to `route_ws` (hm_route_workspace_bytes(tokens, hidden, experts) bytes, 16-byte
- * aligned).  With route_ws given, the logit sums take a certified parallel
- * form whose partials live in route_ws: FP64 block chains for batches of at
- * most 16 tokens, FP64 matrix-core sums for larger batches when E % 64 == 0
- * and H % 16 == 0.  A logit whose float the error bound does not settle is
- * recomputed by the sequential chain, so the results are those of the
- * sequential form.  `flags`: HM_ROUTE_* bits, optionally
+ * aligned).  Batches of more than 16 tokens run the reference's chain of
+ * every logit on the FP64 matrix cores; with route_ws given, smaller ones
+ * (hidden % 32 == 0) take FP64 block sums whose partials live in route_ws, and
+ * a logit whose float their error bound does not settle is recomputed by the
+ * sequential chain.  `flags`: HM_ROUTE_* bits, optionally
  * HM_EXEC_ROUTE_SEQUENTIAL. */
 size_t hm_route_workspace_bytes(int64_t tokens, int64_t hidden, int64_t experts);
 int hm_router_topk(const float* h, const float* w, int64_t tokens,

@@ -208,6 +208,83 @@ def test_router_parallel_nonfinite_sets_status(dev, T, E):
     assert (g["ids"] < E).all()
 
 
+# the batch chain kernel: 4, 8, 16 and 32 tokens a workgroup (by token and
+# expert count) with 16- and 4-byte W loads; K of one partial stage, whole
+# stages, and a remainder; expert counts around 64; tokens off the workgroup's
+BATCH_CASES = [(17, 64, 1, 1, 1, 1), (18, 96, 63, 5, 1, 1), (19, 1024, 65, 6, 1, 0), (21, 2560, 60, 8, 1, 1),
+               (130, 800, 200, 8, 0, 0), (40, 320, 1000, 16, 1, 1), (700, 2048, 128, 8, 1, 1),
+               (1100, 64, 64, 4, 1, 1), (2040, 96, 128, 8, 1, 1), (1300, 33, 130, 4, 1, 1),
+               (4095, 100, 128, 8, 1, 1), (2700, 70, 130, 8, 1, 1)]
+
+
+@pytest.mark.parametrize("T,H,E,k,sm,rn", BATCH_CASES)
+def test_router_batch_bitexact(dev, T, H, E, k, sm, rn):
+    """The reference's chains of a whole batch side by side: logits, ids, scores
+    and groups bit-exact, from rows and router weights off 16-byte alignment
+    too, and with the flag that asks for the sequential chain."""
+    from hmoe import capi
+    print(f"[gpu] router batch T={T} H={H} E={E} k={k}", flush=True)
+    rng = np.random.default_rng(T + H + E)
+    h = O.rmsnorm(rng.standard_normal((T, H)).astype(np.float32), np.ones(H, np.float32))
+    w = (0.02 * rng.standard_normal((H, E))).astype(np.float32)
+    flags = (1 if sm else 0) | (2 if rn else 0)
+    rc, logits = O.router_logits(h, w)
+    assert rc == 0
+    rc, ids, scores = O.route(h, w, k, sm, rn)
+    counts, offsets, ptok, pw, slots = O.group(ids, scores, E)
+    for extra in (0, capi.HM_EXEC_ROUTE_SEQUENTIAL):
+        g = run_router(dev, h, w, k, flags | extra)
+        assert_bitexact(g["logits"], logits, "logits")
+        assert_bitexact(g["ids"], ids, "ids")
+        assert_bitexact(g["scores"], scores, "scores")
+        assert_bitexact(g["ptok"], ptok, "groups")
+    dh = dev.to(np.concatenate([np.zeros(1, np.float32), h.reshape(-1)]))[1:]
+    dw = dev.to(np.concatenate([np.zeros(1, np.float32), w.reshape(-1)]))[1:]
+    out = dict(ids=dev.empty((T, k), np.int32), scores=dev.empty((T, k), np.float32), status=dev.zeros(1, np.int32))
+    ws = dev.empty(dev.lib.hm_route_workspace_bytes(T, H, E), np.uint8)
+    dev.call("hm_router_topk", dh.data_ptr(), dw.data_ptr(), T, H, E, k, flags, out["ids"].data_ptr(),
+             out["scores"].data_ptr(), None, out["status"].data_ptr(), ws.data_ptr(), dev.stream)
+    assert_bitexact(dev.host(out["ids"], np.uint32), ids, "ids, operands off alignment")
+    assert_bitexact(dev.host(out["scores"]), scores, "scores, operands off alignment")
+
+
+def test_router_batch_boundary_and_nonfinite_logits(dev):
+    """Exact float midpoints and cancellations in a batch, and a non-finite
+    score."""
+    T, E, H = 1100, 64, 512
+    rng = np.random.default_rng(4)
+    h = rng.standard_normal((T, H)).astype(np.float32)
+    w = (0.02 * rng.standard_normal((H, E))).astype(np.float32)
+    h[:3] = 0
+    h[0, 0], h[0, 1] = 1.0, 2.0 ** -24
+    w[0, :40], w[1, :40] = 1.0, 1.0          # 40 logits of token 0: 1 + 2^-24 -> 1.0
+    h[1, 0], h[1, 500] = 1.0, 1.0
+    w[0, 50], w[500, 50] = 0.375, -0.375     # token 1, expert 50: exactly 0
+    g = run_router(dev, h, w, 2, 3)
+    rc, logits = O.router_logits(h, w)
+    assert rc == 0
+    assert_bitexact(g["logits"], logits, "logits at rounding boundaries")
+    assert g["logits"][0, 0] == 1.0 and g["logits"][1, 50] == 0.0
+    w[3, 5] = np.inf
+    bad = run_router(dev, h, w, 2, 3)
+    assert bad["status"] & 1 and (bad["ids"] < E).all()
+
+
+@pytest.mark.parametrize("T,E", [(20, 40), (700, 128), (2040, 128), (4000, 128)])
+def test_router_batch_wide_exponents(dev, T, E):
+    """Operands over 2^40 in magnitude at every workgroup form: the matrix
+    instructions' order and roundings of the k terms show in the logits, which
+    equal the reference's chains bit for bit."""
+    H = 192
+    rng = np.random.default_rng(T)
+    h = (rng.standard_normal((T, H)) * np.exp2(rng.integers(-20, 20, (T, H)))).astype(np.float32)
+    w = (rng.standard_normal((H, E)) * np.exp2(rng.integers(-20, 20, (H, E)))).astype(np.float32)
+    g = run_router(dev, h, w, 2, 0)
+    rc, logits = O.router_logits(h, w)
+    assert rc == 0
+    assert_bitexact(g["logits"], logits, "logits")
+
+
 def test_permute_invariants_large(dev):
     """C4 shape (T=4096, E=128, k=8) with Zipf-skewed routing: permutation
     bit-exact against the oracle grouping of the oracle's routing."""
