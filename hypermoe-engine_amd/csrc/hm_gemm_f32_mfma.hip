@@ -1,23 +1,41 @@
-// hm_gemm_f32_mfma.hip -- grouped FP32-weight expert GEMMs on the FP32
-// matrix cores (v_mfma_f32_32x32x2_f32) for gfx950: the A5' path
+// hm_gemm_f32_mfma.hip -- grouped FP32-weight expert GEMMs on the bf16 matrix
+// cores (v_mfma_f32_16x16x32_bf16) for gfx950: the A5' path
 // (ExpertExecutor.cpp:97-131 on CpuTensorBackend::matmul, :87-131).
 //
-// The reference sums each output sequentially in FP32; here the K terms are
-// summed by the matrix cores in an order of their own, so the results are
-// within the FP32 path's 1e-3 of the reference, not bit-identical (the same
-// contract as the FMA tiles in hm_gemm.hip, which remain for other shapes).
+// Every FP32 operand is cut into three bf16 parts of eight bits each, whose
+// sum is the operand exactly (each the top 16 bits of what the parts before it
+// leave), and a product x w is the six products of parts x_i w_j with i + j <=
+// 4: each exact, what is left out below 2^-21 |x w|, and the sums in FP32.  The
+// error against 64-bit sums is smaller than that of FP32 matrix instructions
+// on the whole values (an expert's output at K = 2048, 768: 4.8e-7 against
+// 1.3e-6), as these round once per two k, the split ones' leading sums once per
+// 32.  The reference sums each
+// output sequentially in FP32: the results are within the FP32 path's 1e-3 of
+// it, not bit-identical (as the FMA tiles in hm_gemm.hip, which remain for
+// other shapes).  An operand that is not finite gives NaN parts; such outputs
+// are summed again as the reference does.
+//
+// What bounds them: reading the weights (1.2 GB at 64 experts: 230 us at a large
+// copy's rate) once the matrix work fits under it.  FP32 MFMA does not (157
+// TFLOP/s: 250 us for 512 tokens, 380 with its 64-row tiles' padding); six bf16
+// products take 3/8 of its cycles, and the cutting (5.5 vector instructions an
+// element) about as much again, beside them.  Measured at 512 tokens, 64
+// experts top-8: gate/up 409 -> 315 us, down 190 -> 159 us (70 % of the vector
+// issue).
 //
 // Workgroup: 4 waves, tile BM = 64 grouped rows x 128 weight rows (gate/up:
-// 64 gate + the same 64 up columns; down: 128 output columns).  Wave (wr,
-// wc) owns rows 32*wr .. +31 and two 32-column MFMA accumulators (gate/up:
-// the gate and the up block of columns 32*wc; down: columns 64*wc and
-// 64*wc + 32).  K moves in stages of 32 floats through a 3-slot LDS ring
-// filled by 16-byte direct loads (global_load_lds).  Lane (g, i) =
-// (lane/32, lane%32) supplies A = x[row i][k] and B = W[col i][k]; with a
-// float4 of each per lane, MFMA step j of a group of four takes
-// k = 8q + 4g + j, so every lane reads 16 contiguous bytes per four MFMAs.
-// Rows of a stage are 128 bytes; the 16-byte chunk c of row r is stored at
-// slot c ^ (r % 8), which spreads a reader's 32 rows over the LDS banks.
+// 64 gate + the same 64 up columns; down: 128 output columns).  Wave c owns
+// 32 of the weight rows (gate/up: 16 gate and the 16 up columns beside them)
+// for every 16-row fragment that holds a row, so that a partial tile costs its
+// fragments and no wave waits for another.  K moves in stages of 32 floats
+// through a 3-slot LDS ring filled by 16-byte direct loads (global_load_lds);
+// two workgroups fit a CU.  Lane (g, i) = (lane/16, lane%16) supplies row or
+// column i, k = 8 g .. 8 g + 7 of the stage.  Rows of a stage are 128 bytes; the
+// 16-byte chunk c of row r is stored at slot c ^ (r % 8), which spreads a
+// reader's rows over the LDS banks.  Tiles are numbered row tile major, column
+// block minor, in eight contiguous ranges, one per XCD (workgroup i runs on XCD
+// i % 8): the row tiles of one expert read its weights at about the same time
+// from one L2.
 #include "hm_device.h"
 #include "hm_lds_dma.h"
 
@@ -27,120 +45,182 @@ namespace {
 
 constexpr int kFThreads = 256;
 constexpr int kFBM = 64;            // grouped rows per tile
+constexpr int kFRF = kFBM / 16;     // 16-row fragments
 constexpr int kFBN = 128;           // weight rows per tile
 constexpr int kFBK = 32;            // K floats per stage
 constexpr int kFSlots = 3;
 constexpr int kFRow = kFBK * 4;     // bytes per staged row
 constexpr int kFStage = (kFBM + kFBN) * kFRow;  // 24 KB
 
-typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ v16f mfma_f32(float a, float b, v16f c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+// Eight floats (two LDS chunks) as three bf16 vectors whose sum is exactly
+// them.
+__device__ __forceinline__ void split_bf16(const f4& lo, const f4& hi, bf8 (&p)[3]) {
+    uint32_t o[3][4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        uint32_t a[2], b[2], c[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float v = h < 2 ? lo[2 * h + e] : hi[2 * (h - 2) + e];
+            a[e] = __builtin_bit_cast(uint32_t, v);
+            const float r = v - __builtin_bit_cast(float, a[e] & 0xffff0000u);
+            b[e] = __builtin_bit_cast(uint32_t, r);
+            c[e] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, b[e] & 0xffff0000u));
+        }
+        o[0][h] = __builtin_amdgcn_perm(a[1], a[0], 0x07060302u);
+        o[1][h] = __builtin_amdgcn_perm(b[1], b[0], 0x07060302u);
+        o[2][h] = __builtin_amdgcn_perm(c[1], c[0], 0x07060302u);
+    }
+#pragma unroll
+    for (int l = 0; l < 3; ++l) p[l] = __builtin_bit_cast(bf8, make_uint4(o[l][0], o[l][1], o[l][2], o[l][3]));
+}
+
+// Row tiles of every expert (ceil(count / kFBM)).  Every lane of the wave must
+// be active.
+__device__ __forceinline__ int64_t total_tiles(const int32_t* __restrict__ counts, int64_t experts) {
+    int64_t n = 0;
+    for (int64_t e = threadIdx.x & (HM_WAVE - 1); e < experts; e += HM_WAVE)
+        n += ((int64_t)counts[e] + kFBM - 1) / kFBM;
+#pragma unroll
+    for (int d = 1; d < HM_WAVE; d <<= 1) n += __shfl_xor(n, d, HM_WAVE);
+    return n;
 }
 
 // GATEUP: z[g, n] = silu(x_g . Wg[n]) * (x_g . Wu[n]), x_g = hidden[perm[g]],
 // n in [0, I); tile columns n0 .. n0+63.  DOWN: y[g, n] = z_g . Wd[n],
-// n in [0, H); tile columns n0 .. n0+127.
+// n in [0, H); tile columns n0 .. n0+127.  nbn: column blocks.
 template <bool GATEUP>
 __global__ __launch_bounds__(kFThreads) void expert_f32_mfma_kernel(
     const float* __restrict__ x, int K, int N, int experts, const float* __restrict__ packed,
     int hidden, int inter, const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
-    const int32_t* __restrict__ perm_tokens, float* __restrict__ out) {
+    const int32_t* __restrict__ perm_tokens, int nbn, float* __restrict__ out) {
     __shared__ __attribute__((aligned(1024))) char ring[kFSlots][kFStage];
     __shared__ int s_src[kFBM];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave >> 1, wc = wave & 1;
+    // the workgroup's tile (uniform)
+    const int64_t total = total_tiles(counts, experts) * nbn, per = (total + 7) / 8;
+    const int64_t idx = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per || idx >= total) return;
     int64_t e64, mt;
-    if (!hm_locate_tile(counts, experts, kFBM, blockIdx.x, &e64, &mt)) return;
+    if (!hm_locate_tile(counts, experts, kFBM, idx / nbn, &e64, &mt)) return;
     const int e = (int)e64;
     const int64_t g0 = offsets[e] + mt * kFBM;
-    const int rows = (int)min((int64_t)kFBM, (int64_t)counts[e] - mt * kFBM);
-    const int64_t n0 = (int64_t)blockIdx.y * (GATEUP ? kFBN / 2 : kFBN);
+    const int rows = __builtin_amdgcn_readfirstlane((int)min((int64_t)kFBM, (int64_t)counts[e] - mt * kFBM));
+    const int64_t n0 = (idx % nbn) * (GATEUP ? kFBN / 2 : kFBN);
     if (tid < kFBM) {
         const int r = tid < rows ? tid : rows - 1;  // rows past the group repeat its last
         s_src[tid] = GATEUP ? perm_tokens[g0 + r] : (int)(g0 + r);
     }
     __syncthreads();
-    // this wave's DMA rows: activation rows 16*wave .. +15 (2 loads), weight
-    // rows 32*wave .. +31 (4 loads); lane l covers row base + l/8, slot l%8
+    // this wave's DMA rows: activation rows 16*wave .. +15 (2 loads, none
+    // where the fragment holds no row), weight rows 32*wave .. +31 (4 loads);
+    // lane l covers row base + l/8, slot l%8
+    const bool aload = 16 * wave < rows;
     const int slot = lane & 7, rsub = lane >> 3;
     const float* asrc[2];
     for (int i = 0; i < 2; ++i) {
         const int r = 16 * wave + 8 * i + rsub;
-        const int c = slot ^ (r & 7);
-        asrc[i] = x + (int64_t)s_src[r] * K + 4 * c;
+        asrc[i] = x + (int64_t)s_src[r] * K + 4 * (slot ^ (r & 7));
     }
     const float* wbase = packed + (int64_t)e * 3 * hidden * inter;
     const float* wsrc[4];
     for (int i = 0; i < 4; ++i) {
         const int r = 32 * wave + 8 * i + rsub;  // 0 .. 127
-        const int c = slot ^ (r & 7);
-        int64_t row;
-        const float* proj;
-        if (GATEUP) {
-            proj = wbase + (int64_t)(r >= 64 ? 1 : 0) * hidden * inter;
-            row = n0 + (r & 63);
-        } else {
-            proj = wbase + 2 * (int64_t)hidden * inter;
-            row = n0 + r;
-        }
-        wsrc[i] = proj + row * K + 4 * c;
+        const float* proj = wbase + (int64_t)(GATEUP ? (r >= 64 ? 1 : 0) : 2) * hidden * inter;
+        wsrc[i] = proj + (n0 + (GATEUP ? r & 63 : r)) * K + 4 * (slot ^ (r & 7));
     }
     const int nk = K / kFBK;
     auto issue = [&](int sl, int ks) {
         char* st = ring[sl];
         const int64_t k0 = (int64_t)ks * kFBK;
-        for (int i = 0; i < 2; ++i) dma16(asrc[i] + k0, st + (16 * wave + 8 * i) * kFRow);
         for (int i = 0; i < 4; ++i)
             dma16(wsrc[i] + k0, st + kFBM * kFRow + (32 * wave + 8 * i) * kFRow);
+        if (aload)
+            for (int i = 0; i < 2; ++i) dma16(asrc[i] + k0, st + (16 * wave + 8 * i) * kFRow);
     };
-    v16f acc0 = {}, acc1 = {};
-    const int g = lane >> 5, li = lane & 31;
-    // this lane's rows in the stage: activation row 32*wr + li; weight rows
-    // (gate/up) 32*wc + li and 64 + 32*wc + li, (down) 64*wc + li, +32
-    const int ar = 32 * wr + li;
-    const int br0 = GATEUP ? 32 * wc + li : 64 * wc + li;
-    const int br1 = GATEUP ? 64 + 32 * wc + li : 64 * wc + 32 + li;
+    // the sums of the first parts' products, and of the five others' (2^-8 of
+    // them: their roundings do not count), apart
+    f4 acc[kFRF][2], low[kFRF][2];
+#pragma unroll
+    for (int r = 0; r < kFRF; ++r) acc[r][0] = acc[r][1] = low[r][0] = low[r][1] = f4{};
+    const int g = lane >> 4, li = lane & 15;
+    // this lane's weight rows of the stage: (gate/up) 16*wave + li and
+    // 64 + 16*wave + li, (down) 32*wave + li, +16; all of them li mod 8
+    const int b0 = GATEUP ? 16 * wave + li : 32 * wave + li;
+    const int b1 = b0 + (GATEUP ? 64 : 16);
+    const int c0 = 16 * ((2 * g) ^ (li & 7)), c1 = 16 * ((2 * g + 1) ^ (li & 7));
     issue(0, 0);
     if (nk > 1) issue(1, 1);
     for (int ks = 0; ks < nk; ++ks) {
-        if (ks + 1 < nk) wait_vmcnt<6>();
-        else wait_vmcnt<0>();
+        if (ks + 1 >= nk) wait_vmcnt<0>();
+        else if (aload) wait_vmcnt<6>();
+        else wait_vmcnt<4>();
         lds_barrier();  // stage ks landed for every wave; stage ks-1 fully read
         if (ks + 2 < nk) issue((ks + 2) % kFSlots, ks + 2);
         const char* st = ring[ks % kFSlots];
-        const char* arow = st + ar * kFRow;
-        const char* b0row = st + kFBM * kFRow + br0 * kFRow;
-        const char* b1row = st + kFBM * kFRow + br1 * kFRow;
+        const char* wst = st + kFBM * kFRow;
+        bf8 wp[2][3];
+        split_bf16(*reinterpret_cast<const f4*>(wst + b0 * kFRow + c0),
+                   *reinterpret_cast<const f4*>(wst + b0 * kFRow + c1), wp[0]);
+        split_bf16(*reinterpret_cast<const f4*>(wst + b1 * kFRow + c0),
+                   *reinterpret_cast<const f4*>(wst + b1 * kFRow + c1), wp[1]);
 #pragma unroll
-        for (int q = 0; q < kFBK / 8; ++q) {
-            const int c = 2 * q + g;  // 16-byte chunk of k = 8q + 4g .. +3
-            const float4 a = *reinterpret_cast<const float4*>(arow + 16 * (c ^ (ar & 7)));
-            const float4 b0 = *reinterpret_cast<const float4*>(b0row + 16 * (c ^ (br0 & 7)));
-            const float4 b1 = *reinterpret_cast<const float4*>(b1row + 16 * (c ^ (br1 & 7)));
-            acc0 = mfma_f32(a.x, b0.x, acc0);
-            acc1 = mfma_f32(a.x, b1.x, acc1);
-            acc0 = mfma_f32(a.y, b0.y, acc0);
-            acc1 = mfma_f32(a.y, b1.y, acc1);
-            acc0 = mfma_f32(a.z, b0.z, acc0);
-            acc1 = mfma_f32(a.z, b1.z, acc1);
-            acc0 = mfma_f32(a.w, b0.w, acc0);
-            acc1 = mfma_f32(a.w, b1.w, acc1);
+        for (int r = 0; r < kFRF; ++r) {
+            if (16 * r >= rows) break;  // (uniform)
+            const char* ast = st + (16 * r + li) * kFRow;
+            bf8 xp[3];
+            split_bf16(*reinterpret_cast<const f4*>(ast + c0), *reinterpret_cast<const f4*>(ast + c1), xp);
+            // the parts' products, the smallest first
+#pragma unroll
+            for (int sum = 2; sum >= 1; --sum)
+#pragma unroll
+                for (int i = sum; i >= 0; --i)
+#pragma unroll
+                    for (int f = 0; f < 2; ++f)
+                        low[r][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[i], wp[f][sum - i], low[r][f], 0, 0, 0);
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+                acc[r][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[0], wp[f][0], acc[r][f], 0, 0, 0);
         }
     }
-    // D[r][c]: r = 8*(v/4) + 4*g + v%4, c = lane%32
+    // D of a fragment: lane (g, i) holds rows 4 g .. 4 g + 3 of column i
+    const float inf = __builtin_inff();
+    auto again = [&](int r, int64_t row) __attribute__((noinline)) -> float {
+        // the reference's sum of grouped row r with weight row `row` of the
+        // expert (gate rows, up rows, down rows back to back)
+        const float* xr = x + (int64_t)s_src[r] * K;
+        const float* wr = wbase + row * K;
+        float s = 0.0f;
+        for (int k = 0; k < K; ++k) s = __fadd_rn(s, __fmul_rn(xr[k], wr[k]));
+        return s;
+    };
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int r = 32 * wr + 8 * (v >> 2) + 4 * g + (v & 3);
-        if (r >= rows) continue;
-        float* orow = out + (g0 + r) * (int64_t)N;
-        if (GATEUP) {
-            orow[n0 + 32 * wc + li] = __fmul_rn(hm_silu(acc0[v]), acc1[v]);
-        } else {
-            orow[n0 + 64 * wc + li] = acc0[v];
-            orow[n0 + 64 * wc + 32 + li] = acc1[v];
+    for (int rf = 0; rf < kFRF; ++rf) {
+        if (16 * rf >= rows) break;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = 16 * rf + 4 * g + v;
+            if (r >= rows) continue;
+            float a0 = __fadd_rn(acc[rf][0][v], low[rf][0][v]);
+            float a1 = __fadd_rn(acc[rf][1][v], low[rf][1][v]);
+            float* orow = out + (g0 + r) * (int64_t)N + n0;
+            if (GATEUP) {
+                const int64_t n = n0 + 16 * wave + li;
+                if (!(fabsf(a0) < inf)) a0 = again(r, n);
+                if (!(fabsf(a1) < inf)) a1 = again(r, inter + n);
+                orow[16 * wave + li] = __fmul_rn(hm_silu(a0), a1);
+            } else {
+                const int64_t n = n0 + 32 * wave + li;
+                const int64_t down = 2 * (int64_t)inter * hidden / K;
+                if (!(fabsf(a0) < inf)) a0 = again(r, down + n);
+                if (!(fabsf(a1) < inf)) a1 = again(r, down + n + 16);
+                orow[32 * wave + li] = a0;
+                orow[32 * wave + 16 + li] = a1;
+            }
         }
     }
 }
@@ -158,12 +238,13 @@ bool hm_f32_mfma_down_ok(int64_t H, int64_t I) {
 int hm_launch_gateup_f32_mfma(const hm_layer* L, const float* hidden, const int32_t* counts,
                               const int32_t* offsets, const int32_t* perm_tokens, int64_t R,
                               int64_t max_tiles, float* z, hipStream_t stream) {
-    if (R > INT_MAX || max_tiles > INT_MAX) return HM_ERR_OVERFLOW;
-    const dim3 grid((unsigned)max_tiles, (unsigned)(L->intermediate / (kFBN / 2)));
+    const int64_t nbn = L->intermediate / (kFBN / 2);
+    if (R > INT_MAX || max_tiles > ((1 << 24) - 8) / nbn) return HM_ERR_OVERFLOW;  // 2^32 threads
+    const dim3 grid((unsigned)((max_tiles * nbn + 7) / 8 * 8));
     HM_STAGE_LAUNCH(true, true, expert_f32_mfma_kernel<true>, grid, dim3(kFThreads), 0, stream,
                     hidden, (int)L->hidden, (int)L->intermediate, (int)L->experts,
                     static_cast<const float*>(L->packed), (int)L->hidden, (int)L->intermediate,
-                    counts, offsets, perm_tokens, z);
+                    counts, offsets, perm_tokens, (int)nbn, z);
     HM_LAUNCHED();
     return HM_OK;
 }
@@ -171,12 +252,13 @@ int hm_launch_gateup_f32_mfma(const hm_layer* L, const float* hidden, const int3
 int hm_launch_down_f32_mfma(const hm_layer* L, const float* z, const int32_t* counts,
                             const int32_t* offsets, int64_t R, int64_t max_tiles, float* y,
                             hipStream_t stream) {
-    if (R > INT_MAX || max_tiles > INT_MAX) return HM_ERR_OVERFLOW;
-    const dim3 grid((unsigned)max_tiles, (unsigned)(L->hidden / kFBN));
+    const int64_t nbn = L->hidden / kFBN;
+    if (R > INT_MAX || max_tiles > ((1 << 24) - 8) / nbn) return HM_ERR_OVERFLOW;  // 2^32 threads
+    const dim3 grid((unsigned)((max_tiles * nbn + 7) / 8 * 8));
     hipLaunchKernelGGL(expert_f32_mfma_kernel<false>, grid, dim3(kFThreads), 0, stream, z,
                        (int)L->intermediate, (int)L->hidden, (int)L->experts,
                        static_cast<const float*>(L->packed), (int)L->hidden,
-                       (int)L->intermediate, counts, offsets, nullptr, y);
+                       (int)L->intermediate, counts, offsets, nullptr, (int)nbn, y);
     HM_LAUNCHED();
     return HM_OK;
 }

@@ -524,6 +524,63 @@ def test_block_one_token_nonfinite_score(dev):
     assert_compare(dev.host(res.output), rout, 1e-4, 1e-4, "output after the failed call")
 
 
+@pytest.mark.parametrize("T,H,E,I,k,skew", [
+    (17, 128, 3, 64, 2, False), (64, 256, 1, 128, 1, False), (65, 128, 1, 64, 1, False),
+    (130, 1024, 4, 192, 1, True), (250, 2048, 16, 768, 4, True)])
+def test_block_fp32_split_tiles(dev, T, H, E, I, k, skew):
+    """FP32 experts on the split bf16 tiles: fragment and tile edges (16, 64, 65
+    rows of an expert, one K stage of slack, fewer tiles than XCDs).  An expert
+    output is two chained sums: within (H + I + 64) 2^-22 of the absolute sums
+    (a product's left-out parts are below 2^-21, each FP32 addition 2^-24)."""
+    print(f"[gpu] fp32 split T={T} H={H} E={E} I={I}", flush=True)
+    payload, scale, zp, h, w = _layer_inputs(5 + T, T, H, E, I, False, skew=skew)
+    block = MoEBlock(DeviceExpertLayer(payload, scale, zp, H, I), k)
+    res = block.execute_batch(dev.to(h), dev.to(w))
+    got = dev.host(res.expert_out).astype(np.float64)
+    P = payload.astype(np.float64)
+    for b in res.batches:
+        x = h[b.token_indices].astype(np.float64)
+        g, u, d = (P[b.expert_id, j].reshape(s) for j, s in enumerate([(H, I), (H, I), (I, H)]))
+        gg, uu = x @ g, x @ u
+        z = gg / (1 + np.exp(-gg)) * uu
+        zabs = (np.abs(x) @ np.abs(g)) * (np.abs(x) @ np.abs(u)) + np.abs(z)
+        lo = res.offsets[b.expert_id]
+        rows = got[lo:lo + len(x)]
+        assert np.all(np.abs(rows - z @ d) <= (H + I + 64) * 2.0 ** -22 * (zabs @ np.abs(d)))
+        err = np.linalg.norm(rows - z @ d) / np.linalg.norm(z @ d)
+        assert err < 1e-6, err
+
+
+def test_block_fp32_nonfinite_values(dev):
+    """Non-finite activations and weights reach exactly the expert outputs that
+    the reference's sums give them (their bf16 parts are no numbers: those sums
+    are redone)."""
+    T, H, E, I, k = 40, 128, 2, 64, 2
+    payload, scale, zp, h, w = _layer_inputs(9, T, H, E, I, False)
+    h = h.copy()
+    w = w.copy()
+    w[3:6] = 0                               # the router does not read the features below
+    h[:, 3:6] = 0.5
+    payload = payload.copy()
+    payload[1, 0].reshape(H, I)[4, 7] = np.inf
+    payload[0, 2].reshape(I, H)[9, 11] = np.nan
+    layer = DeviceExpertLayer(payload, scale, zp, H, I)
+    res = MoEBlock(layer, k).execute_batch(dev.to(h), dev.to(w))
+    got = dev.host(res.expert_out)
+    with np.errstate(all="ignore"):
+        for b in res.batches:
+            x = h[b.token_indices]
+            e = b.expert_id
+            g, u = O.matmul_f32(x, payload[e, 0].reshape(H, I)), O.matmul_f32(x, payload[e, 1].reshape(H, I))
+            ref = O.matmul_f32(O.silu(g) * u, payload[e, 2].reshape(I, H))
+            rows = got[res.offsets[e]:res.offsets[e] + len(x)]
+            assert_bitexact(np.isnan(rows), np.isnan(ref), "NaN outputs")
+            inf = np.isinf(ref)
+            assert_bitexact(rows[inf], ref[inf], "infinite outputs")
+            fine = np.isfinite(ref)
+            assert np.allclose(rows[fine], ref[fine], rtol=1e-4, atol=1e-5)
+
+
 @pytest.mark.parametrize("T", [1, 16, 300])
 def test_block_graph_replay(dev, T):
     """The block's launch sequence captured as one HIP graph (kernels only:
