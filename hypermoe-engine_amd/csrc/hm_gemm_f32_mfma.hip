@@ -20,16 +20,19 @@
 // TFLOP/s: 250 us for 512 tokens, 380 with its 64-row tiles' padding); six bf16
 // products take 3/8 of its cycles, and the cutting (5.5 vector instructions an
 // element) about as much again, beside them.  Measured at 512 tokens, 64
-// experts top-8: gate/up 409 -> 315 us, down 190 -> 159 us (70 % of the vector
-// issue).
+// experts top-8: gate/up 409 -> 290 us, down 190 -> 140 us; the cutting and the
+// matrix work alone take 217 and 115 us, the loads alone 190 and 100, and what is
+// left between is their overlap.  Cutting each activation once for all four
+// waves (through LDS) halved the vector work and changed neither time.
 //
 // Workgroup: 4 waves, tile BM = 64 grouped rows x 128 weight rows (gate/up:
 // 64 gate + the same 64 up columns; down: 128 output columns).  Wave c owns
 // 32 of the weight rows (gate/up: 16 gate and the 16 up columns beside them)
 // for every 16-row fragment that holds a row, so that a partial tile costs its
 // fragments and no wave waits for another.  K moves in stages of 32 floats
-// through a 3-slot LDS ring filled by 16-byte direct loads (global_load_lds);
-// two workgroups fit a CU.  Lane (g, i) = (lane/16, lane%16) supplies row or
+// through a 2-slot LDS ring filled by 16-byte direct loads (global_load_lds), so
+// that three workgroups fit a CU: they cover each other's waits better than a
+// third slot does (gate/up 290 us; three slots, two workgroups 340).  Lane (g, i) = (lane/16, lane%16) supplies row or
 // column i, k = 8 g .. 8 g + 7 of the stage.  Rows of a stage are 128 bytes; the
 // 16-byte chunk c of row r is stored at slot c ^ (r % 8), which spreads a
 // reader's rows over the LDS banks.  Tiles are numbered row tile major, column
@@ -48,7 +51,7 @@ constexpr int kFBM = 64;            // grouped rows per tile
 constexpr int kFRF = kFBM / 16;     // 16-row fragments
 constexpr int kFBN = 128;           // weight rows per tile
 constexpr int kFBK = 32;            // K floats per stage
-constexpr int kFSlots = 3;
+constexpr int kFSlots = 2;
 constexpr int kFRow = kFBK * 4;     // bytes per staged row
 constexpr int kFStage = (kFBM + kFBN) * kFRow;  // 24 KB
 
@@ -93,7 +96,7 @@ __device__ __forceinline__ int64_t total_tiles(const int32_t* __restrict__ count
 // n in [0, I); tile columns n0 .. n0+63.  DOWN: y[g, n] = z_g . Wd[n],
 // n in [0, H); tile columns n0 .. n0+127.  nbn: column blocks.
 template <bool GATEUP>
-__global__ __launch_bounds__(kFThreads) void expert_f32_mfma_kernel(
+__global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
     const float* __restrict__ x, int K, int N, int experts, const float* __restrict__ packed,
     int hidden, int inter, const int32_t* __restrict__ counts, const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ perm_tokens, int nbn, float* __restrict__ out) {
@@ -154,13 +157,10 @@ __global__ __launch_bounds__(kFThreads) void expert_f32_mfma_kernel(
     const int b1 = b0 + (GATEUP ? 64 : 16);
     const int c0 = 16 * ((2 * g) ^ (li & 7)), c1 = 16 * ((2 * g + 1) ^ (li & 7));
     issue(0, 0);
-    if (nk > 1) issue(1, 1);
     for (int ks = 0; ks < nk; ++ks) {
-        if (ks + 1 >= nk) wait_vmcnt<0>();
-        else if (aload) wait_vmcnt<6>();
-        else wait_vmcnt<4>();
+        wait_vmcnt<0>();
         lds_barrier();  // stage ks landed for every wave; stage ks-1 fully read
-        if (ks + 2 < nk) issue((ks + 2) % kFSlots, ks + 2);
+        if (ks + 1 < nk) issue((ks + 1) % kFSlots, ks + 1);
         const char* st = ring[ks % kFSlots];
         const char* wst = st + kFBM * kFRow;
         bf8 wp[2][3];
