@@ -770,9 +770,11 @@ __device__ __forceinline__ void select_token(float (&v)[EPL], const bool (&valid
                                              uint32_t flags, uint32_t* __restrict__ ids,
                                              float* __restrict__ scores, int32_t* status,
                                              float* seq_lds, uint32_t* l_ids = nullptr,
-                                             float* l_scores = nullptr, bool coherent = false) {
+                                             float* l_scores = nullptr, bool coherent = false,
+                                             const unsigned long long* exp2 = kHmExp2Table) {
     // (l_ids, l_scores: optional LDS copies of this token's ids and scores;
-    // coherent: device-scope stores, hm_store_pair)
+    // coherent: device-scope stores, hm_store_pair; exp2: the expf table,
+    // where the caller has it in LDS)
     if (flags & HM_ROUTE_SOFTMAX) {
         float m = -__uint_as_float(0x7f800000u);
 #pragma unroll
@@ -783,7 +785,7 @@ __device__ __forceinline__ void select_token(float (&v)[EPL], const bool (&valid
 #pragma unroll
         for (int j = 0; j < EPL; ++j) {
             if (!valid[j]) continue;
-            v[j] = hm_expf(__fsub_rn(v[j], m));
+            v[j] = hm_expf_t(__fsub_rn(v[j], m), exp2);
             exact = exact && (v[j] == 0.0f || v[j] >= 0x1p-17f);
             part += (double)v[j];
         }
@@ -853,37 +855,28 @@ __device__ __forceinline__ void select_token(float (&v)[EPL], const bool (&valid
     }
 }
 
+// Workgroups 0 .. sel-1 select, four tokens each; the others (xq.digits) cut
+// four tokens' rows into the fixed-point digits of the INT8 expert GEMMs (the
+// block's activation quantisation, one launch fewer).  Both are chains of
+// latencies of one wave per token (loads, reductions), so they run side by side
+// on waves of their own, and expf's table is read from LDS rather than by a
+// gather that waits on memory once per token.  Against one wave doing both in
+// turn (128 experts, top-8, H = 2048, three digits): 61 tokens 10 -> 5.7 us,
+// 333 11.5 -> 7.3, 2048 15 -> 12; 4096 tokens 19 both ways, where the 84 MB of
+// rows read and digits written (16 us at the copy rate) bound it.
 template <int EPL>
 __global__ __launch_bounds__(kBlock) void router_select_kernel(
     const float* __restrict__ logits, int64_t tokens, int64_t experts,
     int32_t top_k, uint32_t flags, uint32_t* __restrict__ ids,
     float* __restrict__ scores, int32_t* status, const float* __restrict__ h, int64_t hidden,
-    hm_row_quant xq, int32_t* __restrict__ hist) {
+    hm_row_quant xq, int32_t* __restrict__ hist, unsigned sel) {
     extern __shared__ float seq_lds[];  // (kBlock/64) * experts floats
+    __shared__ unsigned long long s_exp2[32];
     const int lane = threadIdx.x & (HM_WAVE - 1);
     const int wave = threadIdx.x / HM_WAVE;
-    const int64_t t = (int64_t)blockIdx.x * (kBlock / HM_WAVE) + wave;
-    if (t >= tokens) return;
-    const float* lt = logits + t * experts;
-    float v[EPL];
-    bool valid[EPL];
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) {
-        const int64_t e = lane + (int64_t)HM_WAVE * j;
-        valid[j] = e < experts;
-        v[j] = valid[j] ? lt[e] : 0.0f;
-    }
-    select_token<EPL>(v, valid, lane, wave, t, experts, top_k, flags, ids, scores, status, seq_lds);
-    // The permutation's histogram of each 1024-pair chunk (hm_permute's
-    // count pass): each lane re-reads the id it has just written.  Integer
-    // counts, so the atomics' order does not matter.
-    if (hist && lane < top_k) {
-        const int64_t pr = t * top_k + lane;
-        atomicAdd(&hist[(pr / kPermChunk) * experts + ids[pr]], 1);
-    }
-    // The token's row in fixed-point digits for the INT8 expert GEMMs (the
-    // block's activation quantisation, one launch fewer).
-    if (xq.digits) {
+    if (blockIdx.x >= sel) {
+        const int64_t t = (int64_t)(blockIdx.x - sel) * (kBlock / HM_WAVE) + wave;
+        if (t >= tokens) return;
         const int nv = (int)(hidden / 256);
         const hm_dlay lay = hm_dlay_x(xq.limbs, hidden);
         int8_t* d = xq.digits + t * lay.row;
@@ -894,6 +887,31 @@ __global__ __launch_bounds__(kBlock) void router_select_kernel(
         case 2: hm_quantize_row_wave<2>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
         default: hm_quantize_row_wave<3>(hrow, nv, d, lay, xq.scales + t, ds, tokens); break;
         }
+        return;
+    }
+    const int64_t t = (int64_t)blockIdx.x * (kBlock / HM_WAVE) + wave;
+    const float* lt = logits + min(t, tokens - 1) * experts;
+    float v[EPL];
+    bool valid[EPL];
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+        const int64_t e = lane + (int64_t)HM_WAVE * j;
+        valid[j] = e < experts;
+        v[j] = lt[valid[j] ? e : experts - 1];
+    }
+    hm_load_exp2_table(s_exp2);
+    __syncthreads();
+    if (t >= tokens) return;
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) v[j] = valid[j] ? v[j] : 0.0f;
+    select_token<EPL>(v, valid, lane, wave, t, experts, top_k, flags, ids, scores, status, seq_lds,
+                      nullptr, nullptr, false, s_exp2);
+    // The permutation's histogram of each 1024-pair chunk (hm_permute's
+    // count pass): each lane re-reads the id it has just written.  Integer
+    // counts, so the atomics' order does not matter.
+    if (hist && lane < top_k) {
+        const int64_t pr = t * top_k + lane;
+        atomicAdd(&hist[(pr / kPermChunk) * experts + ids[pr]], 1);
     }
 }
 
@@ -1821,7 +1839,7 @@ __attribute__((visibility("hidden"))) int hm_router_topk_quant(const float* h, c
     if (tokens > (int64_t)1 << 27) return HM_ERR_OVERFLOW;  // 32-bit grids
     float* logits = logits_out ? logits_out : static_cast<float*>(route_ws);
     const int epl = (int)((experts + HM_WAVE - 1) / HM_WAVE);
-    const dim3 sgrid((unsigned)((tokens + 3) / 4));
+    const unsigned sel = (unsigned)((tokens + 3) / 4);
     const size_t seq_bytes = (size_t)(kBlock / HM_WAVE) * experts * sizeof(float);
     if (route_ws && tokens <= kDecodeTokens && hidden % kNB == 0 && hidden <= INT_MAX) {
         // decode: certified block partials, then select over the logits
@@ -1841,10 +1859,11 @@ __attribute__((visibility("hidden"))) int hm_router_topk_quant(const float* h, c
     if (counted) *counted = hc != nullptr;
     const int rc = launch_router_chains(h, w, tokens, hidden, experts, logits, status, hc, hc_n, stream);
     if (rc) return rc;
+    const dim3 sgrid(bq.digits ? 2 * sel : sel);
 #define HM_SELECT(N)                                                                   \
     hipLaunchKernelGGL(router_select_kernel<N>, sgrid, dim3(kBlock), seq_bytes,        \
                        hm_stream(stream), logits, tokens, experts, top_k, flags, ids,  \
-                       scores, status, h, hidden, bq, hc)
+                       scores, status, h, hidden, bq, hc, sel)
     if (epl <= 1) HM_SELECT(1);
     else if (epl <= 2) HM_SELECT(2);
     else if (epl <= 4) HM_SELECT(4);
