@@ -168,31 +168,17 @@ __device__ __forceinline__ unsigned long long hm_wave_max_u64_dpp(unsigned long 
     }
     return m;
 }
-// The same maximum kept in the vector unit to the end: after the row
-// steps, row_bcast:15 hands rows 0 and 2 on to rows 1 and 3 and
-// row_bcast:31 row 1 on to rows 2 and 3 (rows outside the row mask keep
+// Maximum of unsigned words over the wave, kept in the vector unit to the
+// end: after the row steps, row_bcast:15 hands rows 0 and 2 on to rows 1 and
+// 3 and row_bcast:31 row 1 on to rows 2 and 3 (rows outside the row mask keep
 // their own value), so lane 63 holds the wave's maximum.
-__device__ __forceinline__ unsigned long long hm_wave_max_u64_bcast(unsigned long long v) {
+__device__ __forceinline__ unsigned hm_wave_max_u32(unsigned v) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const unsigned long long o = hm_dpp_u64(v, c);
-        v = o > v ? o : v;
-    }
-    {
-        const int lo = (int)(unsigned)(v & 0xffffffffull), hi = (int)(unsigned)(v >> 32);
-        const unsigned olo = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, 0x142, 0xa, 0xf, false);
-        const unsigned ohi = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, 0x142, 0xa, 0xf, false);
-        const unsigned long long o = ((unsigned long long)ohi << 32) | olo;
-        v = o > v ? o : v;
-    }
-    {
-        const int lo = (int)(unsigned)(v & 0xffffffffull), hi = (int)(unsigned)(v >> 32);
-        const unsigned olo = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, 0x143, 0xc, 0xf, false);
-        const unsigned ohi = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, 0x143, 0xc, 0xf, false);
-        const unsigned long long o = ((unsigned long long)ohi << 32) | olo;
-        v = o > v ? o : v;
-    }
-    return hm_readlane_u64(v, HM_WAVE - 1);
+    for (int c = 0; c < 4; ++c)
+        v = max(v, __builtin_bit_cast(unsigned, hm_dpp_f32(__builtin_bit_cast(float, v), c)));
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xa, 0xf, false));
+    v = max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xc, 0xf, false));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, HM_WAVE - 1);
 }
 // Sum of doubles over the wave (row DPP, then the four rows in ascending
 // row order); callers use it only where any summation order gives the
@@ -458,10 +444,9 @@ __host__ __device__ __forceinline__ int64_t hm_proj_offset(int64_t e, int p, int
     return (3 * e + p) * hm_proj_bytes(H, I);
 }
 
-// Float total order key for top-k: larger score first, equal scores (with
-// -0 == +0) broken by the lower expert id; 0 is never a valid key.
-__device__ __forceinline__ unsigned long long hm_rank_key(float v, unsigned int id) {
-    unsigned int u = v == 0.0f ? 0u : __float_as_uint(v);
-    u = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-    return ((unsigned long long)u << 32) | (0xffffffffu - id);
+// Float order key for top-k: a larger score has the larger key, equal scores
+// (with -0 == +0) have the same one.
+__device__ __forceinline__ unsigned hm_rank_key(float v) {
+    const unsigned u = v == 0.0f ? 0u : __float_as_uint(v);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }

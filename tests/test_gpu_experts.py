@@ -475,6 +475,29 @@ def test_block_c4_prefill_properties(dev):
     assert nw < 1e-4
 
 
+@pytest.mark.parametrize("T,E,k", [(2, 64, 32), (13, 70, 5), (3, 22, 22), (16, 128, 8), (16, 200, 13), (16, 64, 64)])
+@pytest.mark.parametrize("int8", [False, True])
+def test_block_decode_groups(dev, T, E, k, int8):
+    """The decode step's grouping by the workgroup that arrives last: 64 pairs,
+    65 and 66, whole and ragged runs of 64, and the most there are (1024), over
+    one to four rows of experts, with the pairs of the popular experts spread
+    over all the runs; bit-exact against the oracle's grouping."""
+    print(f"[gpu] decode groups T={T} E={E} k={k} int8={int8}", flush=True)
+    H, I = 64, 32
+    payload, scale, zp, h, w = _layer_inputs(5 + E, T, H, E, I, int8, skew=True)
+    layer = DeviceExpertLayer(payload, scale if int8 else None, zp if int8 else None, H, I)
+    res = MoEBlock(layer, k).execute_batch(dev.to(h), dev.to(w))
+    rc, ids, scores = O.route(h, w, k, 1, 1)
+    assert rc == 0
+    counts, offsets, ptok, pw, _ = O.group(ids, scores, E)
+    assert_bitexact(res.ids, ids, "ids")
+    assert_bitexact(res.scores, scores, "scores")
+    assert_bitexact(res.counts, counts, "counts")
+    assert_bitexact(res.offsets, offsets, "offsets")
+    assert_bitexact(res.perm_tokens, ptok, "permutation")
+    assert_bitexact(res.perm_weights, pw, "permuted weights")
+
+
 def test_block_one_token_select_at_rounding_boundaries(dev):
     """One token on the GEMV path: every workgroup of the gate/up launch
     redoes the select (select_gateup_kernel).  Logits the bound cannot

@@ -132,6 +132,27 @@ def test_router_ties_and_duplicates(dev, T):
         assert_bitexact(g["scores"], scores, "scores with ties")
 
 
+@pytest.mark.parametrize("T,E,k,sm", [(2, 64, 64, 1), (16, 130, 64, 0), (5, 1, 1, 1), (20, 100, 37, 0),
+                                      (33, 1000, 64, 1)])
+def test_router_equal_scores_and_signed_zeros(dev, T, E, k, sm):
+    """Selections whose scores repeat across the lanes and rows of experts (three
+    values, and +0 beside -0, which rank as equal), down to the last expert."""
+    print(f"[gpu] equal scores T={T} E={E} k={k}", flush=True)
+    H = 64
+    rng = np.random.default_rng(E)
+    h = np.zeros((T, H), np.float32)
+    h[:, 0] = rng.choice([-1.0, 1.0], T)
+    w = np.zeros((H, E), np.float32)
+    w[0] = rng.choice([0.0, 1.0, -1.0], E)   # h * 0 = -0 summed from +0; +-1
+    if E > 4:
+        h[0] = 0.0                           # a token whose every logit is zero
+    g = run_router(dev, h, w, k, sm)
+    rc, ids, scores = O.route(h, w, k, sm, 0)
+    assert rc == 0 and g["status"] == 0
+    assert_bitexact(g["ids"], ids, "ids of equal scores")
+    assert_bitexact(g["scores"], scores, "scores")
+
+
 def test_router_nonfinite_sets_status(dev):
     """CpuRouterBackend.cpp:47 throws on a non-finite score; the device sets
     HM_STATUS_NONFINITE_SCORE."""
