@@ -1898,7 +1898,8 @@ __attribute__((visibility("hidden"))) int hm_router_topk_quant(const float* h, c
     }
     hm_row_quant bq = {nullptr, nullptr, nullptr, 0};
     if (xq && xq->digits && xq->scales && xq->limbs >= 1 && xq->limbs <= 3 && hidden % 256 == 0 &&
-        hidden / 256 <= kHmQuantMaxV && (uintptr_t)xq->digits % 4 == 0 && (uintptr_t)h % 16 == 0)
+        hidden / 256 <= kHmQuantMaxV && (uintptr_t)xq->digits % 4 == 0 && (uintptr_t)h % 16 == 0 &&
+        tokens <= (int64_t)1 << 24)  // (twice the workgroups: 2^31 threads)
         bq = *xq;
     // the chunk histograms of hm_permute, when the caller passes them
     const int64_t chunks = (tokens * top_k + kPermChunk - 1) / kPermChunk;
