@@ -1639,9 +1639,24 @@ static size_t route_logits_bytes(int64_t tokens, int64_t experts) {
     return ((size_t)tokens * (size_t)experts * sizeof(float) + 255) & ~(size_t)255;
 }
 
+// The bytes a caller provides.  A batch with E % 64 == 0 is asked for 8-byte
+// sums of up to eight K ranges, both operands' norms and a copy of W beside the
+// logits, which it no longer fills: the size is part of the interface (callers
+// allocate by it, and the block without allocation accepts batches by it).
 size_t hm_route_workspace_bytes(int64_t tokens, int64_t hidden, int64_t experts) {
     if (tokens < 0 || experts <= 0 || hidden <= 0) return 0;
-    if (tokens > kDecodeTokens) return route_logits_bytes(tokens, experts);
+    if (tokens > kDecodeTokens) {
+        size_t b = route_logits_bytes(tokens, experts);
+        if (experts % HM_WAVE == 0) {
+            const int64_t tiles = ((tokens + 63) / 64) * (experts / HM_WAVE);
+            size_t sp = 1;
+            while (sp < 8 && tiles * (int64_t)sp < 512) sp *= 2;
+            b += sp * ((size_t)tokens * (size_t)experts + (size_t)tokens + (size_t)experts) *
+                     sizeof(double) +
+                 (size_t)experts * (size_t)hidden * sizeof(float);
+        }
+        return b;
+    }
     return route_logits_bytes(tokens, experts) +
            (size_t)tokens * (size_t)experts * kNB * 2 * sizeof(double);
 }

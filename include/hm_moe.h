@@ -133,8 +133,8 @@ int hm_rmsnorm(const float* x, const float* gamma, float* y, int64_t rows,
  * every logit on the FP64 matrix cores; with route_ws given, smaller ones
  * (hidden % 32 == 0) take FP64 block sums whose partials live in route_ws, and
  * a logit whose float their error bound does not settle is recomputed by the
- * sequential chain.  `flags`: HM_ROUTE_* bits, optionally
- * HM_EXEC_ROUTE_SEQUENTIAL. */
+ * sequential chain.  (For larger batches the size counts more than the logits
+ * they use.)  `flags`: HM_ROUTE_* bits, optionally HM_EXEC_ROUTE_SEQUENTIAL. */
 size_t hm_route_workspace_bytes(int64_t tokens, int64_t hidden, int64_t experts);
 int hm_router_topk(const float* h, const float* w, int64_t tokens,
                    int64_t hidden, int64_t experts, int32_t top_k,
