@@ -20,7 +20,7 @@
 // TFLOP/s: 250 us for 512 tokens, 380 with its 64-row tiles' padding); six bf16
 // products take 3/8 of its cycles, and the cutting (5.5 vector instructions an
 // element) about as much again, beside them.  Measured at 512 tokens, 64
-// experts top-8: gate/up 409 -> 290 us, down 190 -> 140 us; the cutting and the
+// experts top-8: gate/up 410 -> 302 us, down 190 -> 147 us; the cutting and the
 // matrix work alone take 217 and 115 us, the loads alone 190 and 100, and what is
 // left between is their overlap.  Cutting each activation once for all four
 // waves (through LDS) halved the vector work and changed neither time.
@@ -32,7 +32,7 @@
 // fragments and no wave waits for another.  K moves in stages of 32 floats
 // through a 2-slot LDS ring filled by 16-byte direct loads (global_load_lds), so
 // that three workgroups fit a CU: they cover each other's waits better than a
-// third slot does (gate/up 290 us; three slots, two workgroups 340).  Lane (g, i) = (lane/16, lane%16) supplies row or
+// third slot does (gate/up 302 us; three slots, two workgroups 340).  Lane (g, i) = (lane/16, lane%16) supplies row or
 // column i, k = 8 g .. 8 g + 7 of the stage.  Rows of a stage are 128 bytes; the
 // 16-byte chunk c of row r is stored at slot c ^ (r % 8), which spreads a
 // reader's rows over the LDS banks.  Tiles are numbered row tile major, column

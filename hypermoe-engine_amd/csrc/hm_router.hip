@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_wave_kernel(
 // of 256 steps, narrow, wide and full double operands, no difference; the
 // other orders differ in three of four).  So with k slot g of step s holding
 // k = 4 s + g, one accumulator from +0 over all of K is the reference's chain:
-// no bound, no fallback, no workspace.
+// no bound, no fallback, nothing kept beside the logits.
 //
 // What bounds it: FP64 matrix rate for many tokens (4096 x 2048 x 128: 27 us),
 // and for few the chain itself: 512 dependent 4 x 4 x 4 steps of 21 cycles (5
@@ -253,10 +253,10 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_wave_kernel(
 //
 // Measured, logits + selection inside a block at H = 2048, E = 128 (before:
 // K ranges summed on the matrix cores, an error bound in the select kernel, and
-// a second sum and chains for what it left open): 61 tokens 16 + 23 -> 21 + 10
-// us, 333 17 + 36 -> 21 + 11 us, 2048 32 + 44 -> 40 + 15 us, 4096 55 + 42 -> 60 +
+// a second sum and chains for what it left open): 61 tokens 16 + 23 -> 20 + 6
+// us, 333 17 + 36 -> 21 + 7 us, 2048 32 + 44 -> 38 + 12 us, 4096 55 + 42 -> 58 +
 // 19 us; 201 tokens of H = 1024, E = 60 (one chain per thread before) 87 + 5 ->
-// 13 + 6 us.
+// 13 + 4 us.
 // ---------------------------------------------------------------------------
 constexpr int kCK = 64;   // k per stage
 constexpr int kCH = 68;   // floats from one token's h to the next in a stage
