@@ -4,26 +4,29 @@
 //
 // Every FP32 operand is cut into three bf16 parts of eight bits each, whose
 // sum is the operand exactly (each the top 16 bits of what the parts before it
-// leave), and a product x w is the six products of parts x_i w_j with i + j <=
-// 4: each exact, what is left out below 2^-21 |x w|, and the sums in FP32.  The
-// error against 64-bit sums is smaller than that of FP32 matrix instructions
-// on the whole values (an expert's output at K = 2048, 768: 4.8e-7 against
-// 1.3e-6), as these round once per two k, the split ones' leading sums once per
-// 32.  The reference sums each
-// output sequentially in FP32: the results are within the FP32 path's 1e-3 of
-// it, not bit-identical (as the FMA tiles in hm_gemm.hip, which remain for
-// other shapes).  An operand that is not finite gives NaN parts; such outputs
-// are summed again as the reference does.
+// leave), and a product x w is the eight products of parts other than the two
+// last ones': each exact, what is left out below 2^-32 |x w|, and the sums in
+// FP32.  A single product is thus rounded once, as an FP32 matrix instruction
+// rounds it (six products, without the second part times the third, leave out
+// up to 2^-21 |x w|).  Long sums have a smaller error against 64-bit sums than
+// those of FP32 matrix instructions on the whole values (an expert's output at
+// K = 2048, 768: 4.6e-7 against 1.3e-6), as these round once per two k, the
+// split ones' leading sums once per 32.  The reference sums each output
+// sequentially in FP32: the results are within the FP32 path's 1e-3 of it, not
+// bit-identical (as the FMA tiles in hm_gemm.hip, which remain for other
+// shapes).  An operand that is not finite gives NaN parts; such outputs are
+// summed again as the reference does.
 //
 // What bounds them: reading the weights (1.2 GB at 64 experts: 230 us at a large
 // copy's rate) once the matrix work fits under it.  FP32 MFMA does not (157
-// TFLOP/s: 250 us for 512 tokens, 380 with its 64-row tiles' padding); six bf16
-// products take 3/8 of its cycles, and the cutting (5.5 vector instructions an
-// element) about as much again, beside them.  Measured at 512 tokens, 64
-// experts top-8: gate/up 410 -> 302 us, down 190 -> 147 us; the cutting and the
-// matrix work alone take 217 and 115 us, the loads alone 190 and 100, and what is
-// left between is their overlap.  Cutting each activation once for all four
-// waves (through LDS) halved the vector work and changed neither time.
+// TFLOP/s: 250 us for 512 tokens, 380 with its 64-row tiles' padding); eight bf16
+// products take half of its cycles, and the cutting (5.5 vector instructions an
+// element) somewhat more, beside them.  Measured at 512 tokens, 64 experts
+// top-8: gate/up 410 -> 323 us, down 190 -> 161 us (six products: 296 and 146).
+// With six products the cutting and the matrix work alone took 217 and 115 us,
+// the loads alone 190 and 100, and what was left between was their overlap;
+// cutting each activation once for all four waves (through LDS) halved the
+// vector work and changed neither time.
 //
 // Workgroup: 4 waves, tile BM = 64 grouped rows x 128 weight rows (gate/up:
 // 64 gate + the same 64 up columns; down: 128 output columns).  Wave c owns
@@ -145,7 +148,7 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
         if (aload)
             for (int i = 0; i < 2; ++i) dma16(asrc[i] + k0, st + (16 * wave + 8 * i) * kFRow);
     };
-    // the sums of the first parts' products, and of the five others' (2^-8 of
+    // the sums of the first parts' products, and of the seven others' (2^-7 of
     // them: their roundings do not count), apart
     f4 acc[kFRF][2], low[kFRF][2];
 #pragma unroll
@@ -176,9 +179,9 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
             split_bf16(*reinterpret_cast<const f4*>(ast + c0), *reinterpret_cast<const f4*>(ast + c1), xp);
             // the parts' products, the smallest first
 #pragma unroll
-            for (int sum = 2; sum >= 1; --sum)
+            for (int sum = 3; sum >= 1; --sum)
 #pragma unroll
-                for (int i = sum; i >= 0; --i)
+                for (int i = min(sum, 2); i >= max(0, sum - 2); --i)
 #pragma unroll
                     for (int f = 0; f < 2; ++f)
                         low[r][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[i], wp[f][sum - i], low[r][f], 0, 0, 0);

@@ -604,6 +604,35 @@ def test_block_fp32_nonfinite_values(dev):
             assert np.allclose(rows[fine], ref[fine], rtol=1e-4, atol=1e-5)
 
 
+def _one_term_layer(t, d):
+    """One FP32 expert of H = len(d), I = 64 for one-hot rows: feature r gives
+    the intermediate value t[r] in column 0 (silu(32) = 32 times t[r] / 32) and 0
+    in the others, and the output is the single product t[r] * d[n]."""
+    H, I = len(d), 64
+    payload = np.zeros((1, 3, H * I), np.float32)
+    payload[0, 0].reshape(H, I)[:, 0] = 32.0
+    payload[0, 1].reshape(H, I)[:, 0] = t / np.float32(32.0)
+    payload[0, 2].reshape(I, H)[0] = d
+    return DeviceExpertLayer(payload, None, None, H, I)
+
+
+def test_block_fp32_one_term_sums(dev):
+    """An expert sum of a single product is that product, rounded once: a
+    product's parts left out and the small parts' own roundings are below 2^-6
+    of a rounding.  Values with all 24 bits, among them those whose low parts
+    are largest."""
+    T = H = 128
+    rng = np.random.default_rng(12)
+    t = (1 + rng.random(H)).astype(np.float32)
+    d = (1 + rng.random(H)).astype(np.float32) * rng.choice([-1, 1], H).astype(np.float32)
+    t[:2], d[:2] = np.float32(1 + 2.0 ** -7 - 2.0 ** -23), np.float32(1 + 2.0 ** -7 - 2.0 ** -23)
+    t[2:4], d[2:4] = np.float32(1 + 2.0 ** -8 - 2.0 ** -16), np.float32(-1 - 2.0 ** -8 + 2.0 ** -23)
+    w = rng.standard_normal((H, 1)).astype(np.float32)
+    res = MoEBlock(_one_term_layer(t, d), 1).execute_batch(dev.to(np.eye(T, H, dtype=np.float32)), dev.to(w))
+    exact = t.astype(np.float64)[:, None] * d.astype(np.float64)
+    assert np.all(np.abs(dev.host(res.expert_out) - exact) <= 2.0 ** -24 * (1 + 2.0 ** -6) * np.abs(exact))
+
+
 @pytest.mark.parametrize("T", [1, 16, 300])
 def test_block_graph_replay(dev, T):
     """The block's launch sequence captured as one HIP graph (kernels only:
