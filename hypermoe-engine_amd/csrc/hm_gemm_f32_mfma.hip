@@ -2,31 +2,33 @@
 // cores (v_mfma_f32_16x16x32_bf16) for gfx950: the A5' path
 // (ExpertExecutor.cpp:97-131 on CpuTensorBackend::matmul, :87-131).
 //
-// Every FP32 operand is cut into three bf16 parts of eight bits each, whose
-// sum is the operand exactly (each the top 16 bits of what the parts before it
-// leave), and a product x w is the eight products of parts other than the two
-// last ones': each exact, what is left out below 2^-32 |x w|, and the sums in
-// FP32.  A single product is thus rounded once, as an FP32 matrix instruction
-// rounds it (six products, without the second part times the third, leave out
-// up to 2^-21 |x w|).  Long sums have a smaller error against 64-bit sums than
+// Every FP32 operand times 2^16 is cut into three bf16 parts of eight bits
+// each, whose sum is it exactly (each the top 16 bits of what the parts before
+// it leave; bf16 ends at 2^-133, so without the factor the last bits of
+// operands below 2^-110 would be lost), and a product x w is the eight products
+// of parts other than the two last ones': each exact, what is left out below
+// 2^-32 |x w|, and the sums in FP32.  A single product is thus rounded once, as
+// an FP32 matrix instruction rounds it (six products, without the second part
+// times the third, leave out up to 2^-21 |x w|).  Long sums have a smaller error against 64-bit sums than
 // those of FP32 matrix instructions on the whole values (an expert's output at
 // K = 2048, 768: 4.6e-7 against 1.3e-6), as these round once per two k, the
 // split ones' leading sums once per 32.  The reference sums each output
 // sequentially in FP32: the results are within the FP32 path's 1e-3 of it, not
 // bit-identical (as the FMA tiles in hm_gemm.hip, which remain for other
-// shapes).  An operand that is not finite gives NaN parts; such outputs are
-// summed again as the reference does.
+// shapes).  An operand that is not finite gives NaN parts, one of 2^112 and
+// more or a sum of 2^96 and more infinite ones; such outputs are summed again
+// as the reference does.
 //
 // What bounds them: reading the weights (1.2 GB at 64 experts: 230 us at a large
 // copy's rate) once the matrix work fits under it.  FP32 MFMA does not (157
 // TFLOP/s: 250 us for 512 tokens, 380 with its 64-row tiles' padding); eight bf16
-// products take half of its cycles, and the cutting (5.5 vector instructions an
+// products take half of its cycles, and the cutting (6.5 vector instructions an
 // element) somewhat more, beside them.  Measured at 512 tokens, 64 experts
-// top-8: gate/up 410 -> 323 us, down 190 -> 161 us (six products: 296 and 146).
-// With six products the cutting and the matrix work alone took 217 and 115 us,
-// the loads alone 190 and 100, and what was left between was their overlap;
-// cutting each activation once for all four waves (through LDS) halved the
-// vector work and changed neither time.
+// top-8: gate/up 410 -> 338 us, down 190 -> 169 us (six products: 296 and 146;
+// eight of unscaled operands: 323 and 161).  With six products the cutting and
+// the matrix work alone took 217 and 115 us, the loads alone 190 and 100, and
+// what was left between was their overlap; cutting each activation once for all
+// four waves (through LDS) halved the vector work and changed neither time.
 //
 // Workgroup: 4 waves, tile BM = 64 grouped rows x 128 weight rows (gate/up:
 // 64 gate + the same 64 up columns; down: 128 output columns).  Wave c owns
@@ -61,8 +63,9 @@ constexpr int kFStage = (kFBM + kFBN) * kFRow;  // 24 KB
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
-// Eight floats (two LDS chunks) as three bf16 vectors whose sum is exactly
-// them.
+// Eight floats (two LDS chunks) times 2^16 as three bf16 vectors whose sum is
+// exactly that.
+constexpr float kFScale = 0x1p16f, kFUnscale = 0x1p-32f;
 __device__ __forceinline__ void split_bf16(const f4& lo, const f4& hi, bf8 (&p)[3]) {
     uint32_t o[3][4];
 #pragma unroll
@@ -70,7 +73,7 @@ __device__ __forceinline__ void split_bf16(const f4& lo, const f4& hi, bf8 (&p)[
         uint32_t a[2], b[2], c[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const float v = h < 2 ? lo[2 * h + e] : hi[2 * (h - 2) + e];
+            const float v = kFScale * (h < 2 ? lo[2 * h + e] : hi[2 * (h - 2) + e]);
             a[e] = __builtin_bit_cast(uint32_t, v);
             const float r = v - __builtin_bit_cast(float, a[e] & 0xffff0000u);
             b[e] = __builtin_bit_cast(uint32_t, r);
@@ -208,8 +211,8 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
         for (int v = 0; v < 4; ++v) {
             const int r = 16 * rf + 4 * g + v;
             if (r >= rows) continue;
-            float a0 = __fadd_rn(acc[rf][0][v], low[rf][0][v]);
-            float a1 = __fadd_rn(acc[rf][1][v], low[rf][1][v]);
+            float a0 = kFUnscale * __fadd_rn(acc[rf][0][v], low[rf][0][v]);
+            float a1 = kFUnscale * __fadd_rn(acc[rf][1][v], low[rf][1][v]);
             float* orow = out + (g0 + r) * (int64_t)N + n0;
             if (GATEUP) {
                 const int64_t n = n0 + 16 * wave + li;

@@ -633,6 +633,23 @@ def test_block_fp32_one_term_sums(dev):
     assert np.all(np.abs(dev.host(res.expert_out) - exact) <= 2.0 ** -24 * (1 + 2.0 ** -6) * np.abs(exact))
 
 
+def test_block_fp32_tiny_values(dev):
+    """Operands down to the smallest subnormal keep all their bits in a product
+    of normal size, and operands up to the largest float theirs."""
+    T = H = 128
+    rng = np.random.default_rng(13)
+    t = np.ldexp((1 + rng.random(H)).astype(np.float32), np.arange(H) * 2 - 144)   # 2^-144 .. 2^110
+    t = np.float32(32) * (t / np.float32(32))
+    d = np.ldexp((1 + rng.random(H)).astype(np.float32), 126 - np.arange(H) * 2)   # 2^126 .. 2^-128
+    w = rng.standard_normal((H, 1)).astype(np.float32)
+    res = MoEBlock(_one_term_layer(t, d), 1).execute_batch(dev.to(np.eye(T, H, dtype=np.float32)), dev.to(w))
+    got = dev.host(res.expert_out).astype(np.float64)
+    exact = t.astype(np.float64)[:, None] * d.astype(np.float64)
+    normal = (np.abs(exact) < 2.0 ** 127) & (np.abs(exact) > 2.0 ** -100)
+    assert normal.sum() > H * H // 2
+    assert np.all((np.abs(got - exact) <= 2.0 ** -24 * (1 + 2.0 ** -6) * np.abs(exact))[normal])
+
+
 @pytest.mark.parametrize("T", [1, 16, 300])
 def test_block_graph_replay(dev, T):
     """The block's launch sequence captured as one HIP graph (kernels only:
