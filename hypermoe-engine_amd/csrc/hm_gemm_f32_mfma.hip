@@ -16,15 +16,18 @@
 // sequentially in FP32: the results are within the FP32 path's 1e-3 of it, not
 // bit-identical (as the FMA tiles in hm_gemm.hip, which remain for other
 // shapes).  An operand that is not finite gives NaN parts, one of 2^112 and
-// more or a sum of 2^96 and more infinite ones; such outputs are summed again
-// as the reference does.
+// more or a sum of 2^96 and more infinite ones; a tile with such a sum is
+// summed again on FP32 matrix instructions (v_mfma_f32_16x16x4_f32), which give
+// those outputs what their operands have (512 tokens, 8 experts top-2, H = 1024,
+// I = 512, all of it NaN: the block in 165 us, 107 where it is finite, 4028 with
+// one lane's loop over K for each output).
 //
 // What bounds them: reading the weights (1.2 GB at 64 experts: 230 us at a large
 // copy's rate) once the matrix work fits under it.  FP32 MFMA does not (157
 // TFLOP/s: 250 us for 512 tokens, 380 with its 64-row tiles' padding); eight bf16
 // products take half of its cycles, and the cutting (6.5 vector instructions an
 // element) somewhat more, beside them.  Measured at 512 tokens, 64 experts
-// top-8: gate/up 410 -> 338 us, down 190 -> 169 us (six products: 296 and 146;
+// top-8: gate/up 410 -> 335 us, down 190 -> 161 us (six products: 296 and 146;
 // eight of unscaled operands: 323 and 161).  With six products the cutting and
 // the matrix work alone took 217 and 115 us, the loads alone 190 and 100, and
 // what was left between was their overlap; cutting each activation once for all
@@ -108,18 +111,20 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
     const int32_t* __restrict__ perm_tokens, int nbn, float* __restrict__ out) {
     __shared__ __attribute__((aligned(1024))) char ring[kFSlots][kFStage];
     __shared__ int s_src[kFBM];
+    __shared__ int s_bad;  // a sum of the tile is not finite
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // the workgroup's tile (uniform)
-    const int64_t total = total_tiles(counts, experts) * nbn, per = (total + 7) / 8;
-    const int64_t idx = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
-    if (blockIdx.x / 8 >= per || idx >= total) return;
-    int64_t e64, mt;
-    if (!hm_locate_tile(counts, experts, kFBM, idx / nbn, &e64, &mt)) return;
-    const int e = (int)e64;
-    const int64_t g0 = offsets[e] + mt * kFBM;
-    const int rows = __builtin_amdgcn_readfirstlane((int)min((int64_t)kFBM, (int64_t)counts[e] - mt * kFBM));
-    const int64_t n0 = (idx % nbn) * (GATEUP ? kFBN / 2 : kFBN);
+    // the workgroup's tile (uniform, in scalar registers)
+    const int total = __builtin_amdgcn_readfirstlane((int)total_tiles(counts, experts)) * nbn;
+    const int per = (total + 7) / 8, idx = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= per || idx >= total) return;
+    int64_t e64, mt64;
+    if (!hm_locate_tile(counts, experts, kFBM, idx / nbn, &e64, &mt64)) return;
+    const int e = __builtin_amdgcn_readfirstlane((int)e64), mt = __builtin_amdgcn_readfirstlane((int)mt64);
+    const int64_t g0 = offsets[e] + (int64_t)mt * kFBM;
+    const int rows = min(kFBM, counts[e] - mt * kFBM);
+    const int64_t n0 = (int64_t)(idx % nbn) * (GATEUP ? kFBN / 2 : kFBN);
+    if (tid == 0) s_bad = 0;
     if (tid < kFBM) {
         const int r = tid < rows ? tid : rows - 1;  // rows past the group repeat its last
         s_src[tid] = GATEUP ? perm_tokens[g0 + r] : (int)(g0 + r);
@@ -131,43 +136,47 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
     const bool aload = 16 * wave < rows;
     const int slot = lane & 7, rsub = lane >> 3;
     const float* asrc[2];
+#pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int r = 16 * wave + 8 * i + rsub;
         asrc[i] = x + (int64_t)s_src[r] * K + 4 * (slot ^ (r & 7));
     }
-    const float* wbase = packed + (int64_t)e * 3 * hidden * inter;
-    const float* wsrc[4];
-    for (int i = 0; i < 4; ++i) {
-        const int r = 32 * wave + 8 * i + rsub;  // 0 .. 127
-        const float* proj = wbase + (int64_t)(GATEUP ? (r >= 64 ? 1 : 0) : 2) * hidden * inter;
-        wsrc[i] = proj + (n0 + (GATEUP ? r & 63 : r)) * K + 4 * (slot ^ (r & 7));
-    }
+    // (the weights from a uniform base; a lane's part is the same in each load)
+    const float* wbase = packed + (3 * (int64_t)e + (GATEUP ? wave >> 1 : 2)) * hidden * inter +
+                         (n0 + (GATEUP ? 32 * (wave & 1) : 32 * wave)) * K;
+    const uint32_t woff = 4u * (uint32_t)(rsub * K + 4 * (slot ^ rsub));
     const int nk = K / kFBK;
     auto issue = [&](int sl, int ks) {
         char* st = ring[sl];
         const int64_t k0 = (int64_t)ks * kFBK;
+#pragma unroll
         for (int i = 0; i < 4; ++i)
-            dma16(wsrc[i] + k0, st + kFBM * kFRow + (32 * wave + 8 * i) * kFRow);
+            dma16_off(wbase + 8 * i * (int64_t)K + k0, woff, st + kFBM * kFRow + (32 * wave + 8 * i) * kFRow);
         if (aload)
+#pragma unroll
             for (int i = 0; i < 2; ++i) dma16(asrc[i] + k0, st + (16 * wave + 8 * i) * kFRow);
     };
     // the sums of the first parts' products, and of the seven others' (2^-7 of
     // them: their roundings do not count), apart
     f4 acc[kFRF][2], low[kFRF][2];
-#pragma unroll
-    for (int r = 0; r < kFRF; ++r) acc[r][0] = acc[r][1] = low[r][0] = low[r][1] = f4{};
     const int g = lane >> 4, li = lane & 15;
     // this lane's weight rows of the stage: (gate/up) 16*wave + li and
     // 64 + 16*wave + li, (down) 32*wave + li, +16; all of them li mod 8
     const int b0 = GATEUP ? 16 * wave + li : 32 * wave + li;
     const int b1 = b0 + (GATEUP ? 64 : 16);
     const int c0 = 16 * ((2 * g) ^ (li & 7)), c1 = 16 * ((2 * g + 1) ^ (li & 7));
+#pragma unroll
+    for (int r = 0; r < kFRF; ++r) acc[r][0] = acc[r][1] = low[r][0] = low[r][1] = f4{};
+    // stage ks: landed for every wave, and stage ks-1 fully read
+    auto stage = [&](int ks) __attribute__((always_inline)) {
+        wait_vmcnt<0>();
+        lds_barrier();
+        if (ks + 1 < nk) issue((ks + 1) % kFSlots, ks + 1);
+        return (const char*)ring[ks % kFSlots];
+    };
     issue(0, 0);
     for (int ks = 0; ks < nk; ++ks) {
-        wait_vmcnt<0>();
-        lds_barrier();  // stage ks landed for every wave; stage ks-1 fully read
-        if (ks + 1 < nk) issue((ks + 1) % kFSlots, ks + 1);
-        const char* st = ring[ks % kFSlots];
+        const char* st = stage(ks);
         const char* wst = st + kFBM * kFRow;
         bf8 wp[2][3];
         split_bf16(*reinterpret_cast<const f4*>(wst + b0 * kFRow + c0),
@@ -193,17 +202,53 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
                 acc[r][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[0], wp[f][0], acc[r][f], 0, 0, 0);
         }
     }
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < kFRF; ++r) {
+        if (16 * r >= rows) break;
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                acc[r][f][v] = kFUnscale * __fadd_rn(acc[r][f][v], low[r][f][v]);
+                low[r][f][v] = 0.0f;
+                bad = bad || !(fabsf(acc[r][f][v]) < __builtin_inff());
+            }
+    }
+    if (bad) s_bad = 1;
+    __syncthreads();  // (every stage fully read, too)
+    if (s_bad) {
+        // lane (g, i) holds k = 8 g + 4 q + j in step (q, j)
+        issue(0, 0);
+        for (int ks = 0; ks < nk; ++ks) {
+            const char* st = stage(ks);
+            const char* wst = st + kFBM * kFRow;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int c = q ? c1 : c0;
+                const f4 w0 = *reinterpret_cast<const f4*>(wst + b0 * kFRow + c);
+                const f4 w1 = *reinterpret_cast<const f4*>(wst + b1 * kFRow + c);
+#pragma unroll
+                for (int r = 0; r < kFRF; ++r) {
+                    if (16 * r >= rows) break;  // (uniform)
+                    const f4 xv = *reinterpret_cast<const f4*>(st + (16 * r + li) * kFRow + c);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        low[r][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j], w0[j], low[r][0], 0, 0, 0);
+                        low[r][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[j], w1[j], low[r][1], 0, 0, 0);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kFRF; ++r)
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    acc[r][f][v] = fabsf(acc[r][f][v]) < __builtin_inff() ? acc[r][f][v] : low[r][f][v];
+    }
     // D of a fragment: lane (g, i) holds rows 4 g .. 4 g + 3 of column i
-    const float inf = __builtin_inff();
-    auto again = [&](int r, int64_t row) __attribute__((noinline)) -> float {
-        // the reference's sum of grouped row r with weight row `row` of the
-        // expert (gate rows, up rows, down rows back to back)
-        const float* xr = x + (int64_t)s_src[r] * K;
-        const float* wr = wbase + row * K;
-        float s = 0.0f;
-        for (int k = 0; k < K; ++k) s = __fadd_rn(s, __fmul_rn(xr[k], wr[k]));
-        return s;
-    };
 #pragma unroll
     for (int rf = 0; rf < kFRF; ++rf) {
         if (16 * rf >= rows) break;
@@ -211,21 +256,12 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
         for (int v = 0; v < 4; ++v) {
             const int r = 16 * rf + 4 * g + v;
             if (r >= rows) continue;
-            float a0 = kFUnscale * __fadd_rn(acc[rf][0][v], low[rf][0][v]);
-            float a1 = kFUnscale * __fadd_rn(acc[rf][1][v], low[rf][1][v]);
             float* orow = out + (g0 + r) * (int64_t)N + n0;
             if (GATEUP) {
-                const int64_t n = n0 + 16 * wave + li;
-                if (!(fabsf(a0) < inf)) a0 = again(r, n);
-                if (!(fabsf(a1) < inf)) a1 = again(r, inter + n);
-                orow[16 * wave + li] = __fmul_rn(hm_silu(a0), a1);
+                orow[16 * wave + li] = __fmul_rn(hm_silu(acc[rf][0][v]), acc[rf][1][v]);
             } else {
-                const int64_t n = n0 + 32 * wave + li;
-                const int64_t down = 2 * (int64_t)inter * hidden / K;
-                if (!(fabsf(a0) < inf)) a0 = again(r, down + n);
-                if (!(fabsf(a1) < inf)) a1 = again(r, down + n + 16);
-                orow[32 * wave + li] = a0;
-                orow[32 * wave + 16 + li] = a1;
+                orow[32 * wave + li] = acc[rf][0][v];
+                orow[32 * wave + 16 + li] = acc[rf][1][v];
             }
         }
     }
@@ -233,12 +269,13 @@ __global__ __launch_bounds__(kFThreads, 3) void expert_f32_mfma_kernel(
 
 }  // namespace
 
-// Shapes the FP32 MFMA kernels take (16-byte aligned operands).
+// Shapes the FP32 MFMA kernels take (16-byte aligned operands; eight rows of K
+// floats within a 32-bit offset).
 bool hm_f32_mfma_gateup_ok(int64_t H, int64_t I) {
-    return H % kFBK == 0 && I % (kFBN / 2) == 0 && H <= INT_MAX / 4 && I <= INT_MAX / 4;
+    return H % kFBK == 0 && I % (kFBN / 2) == 0 && H <= (1 << 26) && I <= INT_MAX / 4;
 }
 bool hm_f32_mfma_down_ok(int64_t H, int64_t I) {
-    return I % kFBK == 0 && H % kFBN == 0 && H <= INT_MAX / 4 && I <= INT_MAX / 4;
+    return I % kFBK == 0 && H % kFBN == 0 && H <= INT_MAX / 4 && I <= (1 << 26);
 }
 
 int hm_launch_gateup_f32_mfma(const hm_layer* L, const float* hidden, const int32_t* counts,

@@ -91,6 +91,20 @@ def _op_call(dev, x, w, y, scale=None, zp=0):
              scratch.data_ptr(), scratch.numel() * 4, dev.stream)
 
 
+def _event_ms(call, n=5):
+    import torch
+    call()
+    best = float("inf")
+    for _ in range(n):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        call()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
 @pytest.mark.parametrize("int8", [True, False])
 @pytest.mark.parametrize("rows,inner,cols", OP_SHAPES)
 def test_op_gemm_edges(dev, rows, inner, cols, int8):
@@ -648,6 +662,21 @@ def test_block_fp32_tiny_values(dev):
     normal = (np.abs(exact) < 2.0 ** 127) & (np.abs(exact) > 2.0 ** -100)
     assert normal.sum() > H * H // 2
     assert np.all((np.abs(got - exact) <= 2.0 ** -24 * (1 + 2.0 ** -6) * np.abs(exact))[normal])
+
+
+def test_block_fp32_nonfinite_values_keep_the_speed(dev):
+    """Experts whose every sum is NaN take no more than ten times the time of
+    finite ones (one lane summing over K in turn took hundreds of times)."""
+    T, H, E, I, k = 512, 1024, 8, 512, 2
+    payload, scale, zp, h, w = _layer_inputs(3, T, H, E, I, False)
+    dh, dw = dev.to(h), dev.to(w)
+    bad = payload.copy()
+    bad[:, 0].reshape(E, H, I)[:, 5] = np.nan
+    blocks = [MoEBlock(DeviceExpertLayer(p, scale, zp, H, I), k) for p in (payload, bad)]
+    ms = [_event_ms(lambda: b.launch(dh, dw)) for b in blocks]
+    print(f"[gpu] finite {ms[0]:.3f} ms, NaN {ms[1]:.3f} ms", flush=True)
+    assert np.isnan(dev.host(blocks[1].launch(dh, dw)["expert_out"])).all()
+    assert ms[1] < 10 * ms[0]
 
 
 @pytest.mark.parametrize("T", [1, 16, 300])
