@@ -7,10 +7,12 @@
 //   op_gemm_kernel<int8_t, ..>  y = s (x (q - zp)), bf16 matrix cores
 //                               (v_mfma_f32_16x16x32_bf16): q - zp has at
 //                               most eight significant bits, so it is exact
-//                               in bf16, and x is cut into three bf16 parts
-//                               that hold its 24 bits exactly; the three
-//                               products of a term are exact and only their
-//                               FP32 sums round.
+//                               in bf16, and 2^16 x is cut into three bf16
+//                               parts that hold its 24 bits exactly (bf16
+//                               ends at 2^-133: without the factor the last
+//                               bits of x below 2^-110 would be lost); the
+//                               three products of a term are exact and only
+//                               their FP32 sums round.
 //
 // What bounds them: a call of the sizes an expert's rows have (1 to some
 // hundred rows, K and N up to a few thousand) is 0.01 to 8 GFLOP on a few MB,
@@ -78,9 +80,11 @@ __device__ __forceinline__ uint32_t op_high_halves(float lo, float hi) {
                                  0x07060302u);
 }
 
-// Eight floats as three bf16 vectors whose sum is exactly x: each part the
+// Eight floats as three bf16 vectors whose sum is exactly 2^16 x: each part the
 // top 16 bits of what the parts before it leave (24 = 8 + 8 + 8 bits).  (A
-// non-finite x gives NaN parts; the epilogue redoes such outputs.)
+// non-finite x gives NaN parts, as one of 2^112 and more does; the epilogue
+// redoes such outputs.)
+constexpr float kOpScale = 0x1p16f;
 __device__ __forceinline__ void op_split(const f4 (&x)[2], bf8 (&p)[3]) {
     uint32_t o[3][4];
 #pragma unroll
@@ -88,7 +92,7 @@ __device__ __forceinline__ void op_split(const f4 (&x)[2], bf8 (&p)[3]) {
         float a[2], b[2], c[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const float v = x[h >> 1][2 * (h & 1) + e];
+            const float v = kOpScale * x[h >> 1][2 * (h & 1) + e];
             a[e] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & 0xffff0000u);
             const float r = v - a[e];
             b[e] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xffff0000u);
@@ -105,8 +109,8 @@ __device__ __forceinline__ void op_split(const f4 (&x)[2], bf8 (&p)[3]) {
     }
 }
 
-// x [M x K], w [K x N], y [M x N].  WT = int8_t: y = mant * (the sum with
-// p2-scaled weights), scale = mant * p2; zp the zero point.  WT = float: the
+// x [M x K], w [K x N], y [M x N].  WT = int8_t: y = mant * (the sum of 2^16 x
+// with p2-scaled weights), scale = 2^16 mant p2; zp the zero point.  WT = float: the
 // last four arguments are not read.
 template <typename WT, int RF, int CF, int NW, int D>
 __global__ __launch_bounds__(64 * NW) void op_gemm_kernel(
@@ -366,13 +370,13 @@ int hm_launch_op_gemm_f32(const float* x, const float* w, float* y, int64_t M, i
 // y [M x N] = scale (x [M x K] (q [K x N] - zp)).  The power of two of the
 // scale goes into the weights (q - zp times it is still exact in bf16) and
 // its mantissa into the result, so that no sum is more than a factor of two
-// from the result's own size.
+// from 2^16 times the result's own size.
 int hm_launch_op_gemm_w8a32(const float* x, const int8_t* q, float scale, int32_t zp, float* y,
                             int64_t M, int64_t K, int64_t N, hipStream_t s) {
     int e;
     std::frexp(scale, &e);
     e = e - 1 < -100 ? -100 : e - 1 > 100 ? 100 : e - 1;
-    const float p2 = std::ldexp(1.0f, e), mant = scale / p2;
+    const float p2 = std::ldexp(1.0f, e), mant = scale / p2 / kOpScale;
     switch (op_gemm_tile(kOpTilesI8, M, K, N)) {
     case 0: return op_gemm_launch<int8_t, 1, 2, 16, 2>(x, q, y, M, K, N, zp, p2, mant, scale, s);
     case 1: return op_gemm_launch<int8_t, 1, 4, 8, 2>(x, q, y, M, K, N, zp, p2, mant, scale, s);

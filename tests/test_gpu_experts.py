@@ -163,6 +163,21 @@ def test_op_gemm_special_values(dev, int8):
     assert np.all(np.abs(got - x64 @ w64)[fine] <= bound[fine])
 
 
+def test_op_gemm_tiny_activations(dev):
+    """Activations down to the smallest subnormal keep all their bits (times a
+    scale that brings the results back to the middle of the range): within
+    (K + 32) u sum |x w| of 64-bit sums, as any other row."""
+    M, K, N = 40, 301, 70
+    rng = np.random.default_rng(5)
+    x = (rng.standard_normal((M, K)) * np.exp2(-109.0 - np.arange(M)[:, None])).astype(np.float32)
+    q = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    scale = float(np.float32(0.011) * np.float32(2.0 ** 70))
+    y = dev.empty((M, N), np.float32)
+    _op_call(dev, dev.to(x), dev.to(q), y, scale, 3)
+    x64, w64 = x.astype(np.float64), (q.astype(np.float64) - 3) * scale
+    assert np.all(np.abs(dev.host(y) - x64 @ w64) <= (K + 32) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64)))
+
+
 def test_matmul_f32_closed_form(dev):
     """tests/phase5_tests.cpp:147-160: [[1,2,3],[4,5,6]] x [[7,8],[9,10],[11,12]]."""
     a = np.array([[1, 2, 3], [4, 5, 6]], np.float32)
