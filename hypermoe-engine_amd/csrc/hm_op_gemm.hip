@@ -32,6 +32,8 @@
 
 #include <limits.h>
 
+#include <type_traits>
+
 namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -82,8 +84,8 @@ __device__ __forceinline__ uint32_t op_high_halves(float lo, float hi) {
 
 // Eight floats as three bf16 vectors whose sum is exactly 2^16 x: each part the
 // top 16 bits of what the parts before it leave (24 = 8 + 8 + 8 bits).  (A
-// non-finite x gives NaN parts, as one of 2^112 and more does; the epilogue
-// redoes such outputs.)
+// non-finite x gives NaN parts, as one of 2^112 and more does; such a tile
+// is summed again on the FP32 instructions.)
 constexpr float kOpScale = 0x1p16f;
 __device__ __forceinline__ void op_split(const f4 (&x)[2], bf8 (&p)[3]) {
     uint32_t o[3][4];
@@ -113,7 +115,7 @@ __device__ __forceinline__ void op_split(const f4 (&x)[2], bf8 (&p)[3]) {
 // with p2-scaled weights), scale = 2^16 mant p2; zp the zero point.  WT = float: the
 // last four arguments are not read.
 template <typename WT, int RF, int CF, int NW, int D>
-__global__ __launch_bounds__(64 * NW) void op_gemm_kernel(
+__global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void op_gemm_kernel(
     const float* __restrict__ x, const WT* __restrict__ w, float* __restrict__ y, int64_t M,
     int64_t K, int64_t N, int64_t row_tiles, int64_t tiles, int32_t zp, float p2, float mant,
     float scale) {
@@ -121,11 +123,14 @@ __global__ __launch_bounds__(64 * NW) void op_gemm_kernel(
     typedef typename Step<WT, RF, CF>::type S;
     constexpr int BM = 16 * RF, BN = 16 * CF;
     __shared__ float s_red[NW][BM][BN + 1];
+    __shared__ int s_bad;  // the last tile (1, 2, ..) with an output that is not finite
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, li = lane & 15;
     const int64_t steps = (K + S::K - 1) / S::K;
     const int64_t s0 = wave * steps / NW, s1 = (wave + 1) * steps / NW;
+    if (I8 && tid == 0) s_bad = 0;
+    int round = 0;
     const float bias = I8 ? -(float)(128 + zp) * p2 : 0.0f;
     // Tiles are numbered column block major, row tile minor, in eight
     // contiguous ranges, one per XCD (workgroup i runs on XCD i % 8): the row
@@ -276,34 +281,70 @@ __global__ __launch_bounds__(64 * NW) void op_gemm_kernel(
         }
         // D of a 16 x 16 fragment: lane (g, i) holds rows 4 g .. 4 g + 3 of
         // column i
+        ++round;
+        // (AGAIN: only the outputs that are not finite yet, or all)
+        auto finish = [&](auto again, bool all) __attribute__((always_inline)) {
+            constexpr bool AGAIN = decltype(again)::value;
 #pragma unroll
-        for (int rf = 0; rf < RF; ++rf)
+            for (int rf = 0; rf < RF; ++rf)
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
+                for (int v = 0; v < 4; ++v)
 #pragma unroll
-                for (int f = 0; f < CF; ++f) s_red[wave][16 * rf + 4 * g + v][CF * li + f] = acc[rf][f][v];
-        __syncthreads();
-        for (int u = tid; u < BM * BN; u += 64 * NW) {
-            const int r = u / BN, c = u % BN;
-            if (m0 + r >= M || n0 + c >= N) continue;
-            float sum = s_red[0][r][c];
+                    for (int f = 0; f < CF; ++f) s_red[wave][16 * rf + 4 * g + v][CF * li + f] = acc[rf][f][v];
+            __syncthreads();
+            bool bad = false;
+            for (int u = tid; u < BM * BN; u += 64 * NW) {
+                const int r = u / BN, c = u % BN;
+                if (m0 + r >= M || n0 + c >= N) continue;
+                float* out = y + (m0 + r) * N + n0 + c;
+                if (AGAIN && !all && fabsf(*out) < __builtin_inff()) continue;
+                float sum = s_red[0][r][c];
 #pragma unroll
-            for (int q = 1; q < NW; ++q) sum = __fadd_rn(sum, s_red[q][r][c]);
-            if constexpr (I8) {
-                sum = __fmul_rn(sum, mant);
-                // a non-finite activation (its bf16 parts are NaN) or a sum
-                // past the range: the reference's own loop
-                if (!(fabsf(sum) < __builtin_inff())) {
-                    const float* xr = x + (m0 + r) * K;
-                    const int8_t* wc = reinterpret_cast<const int8_t*>(w) + n0 + c;
-                    sum = 0.0f;
-                    for (int64_t k = 0; k < K; ++k)
-                        sum = __fadd_rn(sum, __fmul_rn(xr[k], __fmul_rn((float)((int)wc[k * N] - zp), scale)));
+                for (int q = 1; q < NW; ++q) sum = __fadd_rn(sum, s_red[q][r][c]);
+                if constexpr (I8 && !AGAIN) {
+                    sum = __fmul_rn(sum, mant);
+                    bad = bad || !(fabsf(sum) < __builtin_inff());
+                }
+                *out = sum;
+            }
+            if (I8 && !AGAIN && bad) s_bad = round;
+            __syncthreads();  // the next sums go to s_red
+        };
+        finish(std::false_type{}, true);
+        if constexpr (I8) {
+            // An output is not finite (an activation that is not, or is 2^112 and
+            // more, or a sum past the range): the tile again on the FP32
+            // instructions, which give such outputs what their operands have, the
+            // weights rounded as the reference rounds them (300 rows of K = 2048,
+            // N = 768, all of it infinite: the call in 44 us, 17 where it is
+            // finite, 444 with one lane's loop over K for each output).
+            if (s_bad != round) continue;  // (uniform)
+#pragma unroll
+            for (int rf = 0; rf < RF; ++rf)
+#pragma unroll
+                for (int f = 0; f < CF; ++f) acc[rf][f] = f4{};
+            const int64_t end = min(s1 * S::K, K);
+#pragma unroll 4
+            for (int64_t k0 = s0 * S::K; k0 < end; k0 += 4) {
+                const int64_t k = min(k0 + g, K - 1);  // both operands are zero past K
+                const bool in = k0 + g < K;
+                float xv[RF];
+#pragma unroll
+                for (int rf = 0; rf < RF; ++rf) {
+                    const float v = xt[min((int64_t)(16 * rf + li), M - 1 - m0) * K + k];
+                    xv[rf] = in ? v : 0.0f;
+                }
+#pragma unroll
+                for (int f = 0; f < CF; ++f) {
+                    const int q = (int)w[k * N + min(nv + f, N - 1)] - zp;
+                    const float wv = __fmul_rn((float)(in ? q : 0), scale);
+#pragma unroll
+                    for (int rf = 0; rf < RF; ++rf)
+                        acc[rf][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[rf], wv, acc[rf][f], 0, 0, 0);
                 }
             }
-            y[(m0 + r) * N + n0 + c] = sum;
+            finish(std::true_type{}, false);
         }
-        __syncthreads();  // the next tile writes s_red
     }
 }
 

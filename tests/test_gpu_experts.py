@@ -178,6 +178,24 @@ def test_op_gemm_tiny_activations(dev):
     assert np.all(np.abs(dev.host(y) - x64 @ w64) <= (K + 32) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64)))
 
 
+def test_op_gemm_nonfinite_rows_keep_the_speed(dev):
+    """Outputs that are not finite come from the matrix cores too: a call whose
+    every output is infinite takes no more than ten times the finite one's time
+    (one lane summing over K in turn took hundreds of times)."""
+    M, K, N = 300, 2048, 768
+    rng = np.random.default_rng(8)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    q, y = dev.to(rng.integers(1, 128, (K, N)).astype(np.int8)), dev.empty((M, N), np.float32)
+    dx = dev.to(x)
+    x[:, 17] = np.inf
+    dinf = dev.to(x)
+    fine = _event_ms(lambda: _op_call(dev, dx, q, y, 0.01))
+    inf = _event_ms(lambda: _op_call(dev, dinf, q, y, 0.01))
+    print(f"[gpu] finite {fine:.3f} ms, infinite {inf:.3f} ms", flush=True)
+    assert np.isposinf(dev.host(y)).all()
+    assert inf < 10 * fine
+
+
 def test_matmul_f32_closed_form(dev):
     """tests/phase5_tests.cpp:147-160: [[1,2,3],[4,5,6]] x [[7,8],[9,10],[11,12]]."""
     a = np.array([[1, 2, 3], [4, 5, 6]], np.float32)
