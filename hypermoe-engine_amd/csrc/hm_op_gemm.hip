@@ -113,12 +113,12 @@ __device__ __forceinline__ void op_split(const f4 (&x)[2], bf8 (&p)[3]) {
 
 // x [M x K], w [K x N], y [M x N].  WT = int8_t: y = mant * (the sum of 2^16 x
 // with p2-scaled weights), scale = 2^16 mant p2; zp the zero point.  WT = float: the
-// last four arguments are not read.
+// last five arguments are not read.
 template <typename WT, int RF, int CF, int NW, int D>
 __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void op_gemm_kernel(
     const float* __restrict__ x, const WT* __restrict__ w, float* __restrict__ y, int64_t M,
     int64_t K, int64_t N, int64_t row_tiles, int64_t tiles, int32_t zp, float p2, float mant,
-    float scale) {
+    float scale, bool past) {
     constexpr bool I8 = sizeof(WT) == 1;
     typedef typename Step<WT, RF, CF>::type S;
     constexpr int BM = 16 * RF, BN = 16 * CF;
@@ -317,8 +317,9 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void op_gemm_kernel(
             // instructions, which give such outputs what their operands have, the
             // weights rounded as the reference rounds them (300 rows of K = 2048,
             // N = 768, all of it infinite: the call in 44 us, 17 where it is
-            // finite, 444 with one lane's loop over K for each output).
-            if (s_bad != round) continue;  // (uniform)
+            // finite, 444 with one lane's loop over K for each output); and every
+            // tile where such weights may be infinite (past).
+            if (s_bad != round && !past) continue;  // (uniform)
 #pragma unroll
             for (int rf = 0; rf < RF; ++rf)
 #pragma unroll
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void op_gemm_kernel(
                         acc[rf][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[rf], wv, acc[rf][f], 0, 0, 0);
                 }
             }
-            finish(std::true_type{}, false);
+            finish(std::true_type{}, past);
         }
     }
 }
@@ -385,12 +386,12 @@ int op_gemm_tile(const OpTile (&tiles)[4], int64_t M, int64_t K, int64_t N) {
 
 template <typename WT, int RF, int CF, int NW, int D>
 int op_gemm_launch(const float* x, const WT* w, float* y, int64_t M, int64_t K, int64_t N,
-                   int32_t zp, float p2, float mant, float scale, hipStream_t s) {
+                   int32_t zp, float p2, float mant, float scale, bool past, hipStream_t s) {
     const int64_t row_tiles = (M + 16 * RF - 1) / (16 * RF);
     const int64_t tiles = row_tiles * ((N + 16 * CF - 1) / (16 * CF));
     const int64_t want = (tiles + 7) / 8 * 8;
     hipLaunchKernelGGL((op_gemm_kernel<WT, RF, CF, NW, D>), dim3((unsigned)(want < (1 << 20) ? want : 1 << 20)),
-                       dim3(64 * NW), 0, s, x, w, y, M, K, N, row_tiles, tiles, zp, p2, mant, scale);
+                       dim3(64 * NW), 0, s, x, w, y, M, K, N, row_tiles, tiles, zp, p2, mant, scale, past);
     HM_LAUNCHED();
     return HM_OK;
 }
@@ -401,10 +402,10 @@ int op_gemm_launch(const float* x, const WT* w, float* y, int64_t M, int64_t K, 
 int hm_launch_op_gemm_f32(const float* x, const float* w, float* y, int64_t M, int64_t K, int64_t N,
                           hipStream_t s) {
     switch (op_gemm_tile(kOpTilesF32, M, K, N)) {
-    case 0: return op_gemm_launch<float, 1, 2, 16, 2>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, s);
-    case 1: return op_gemm_launch<float, 1, 4, 8, 2>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, s);
-    case 2: return op_gemm_launch<float, 2, 4, 4, 4>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, s);
-    default: return op_gemm_launch<float, 4, 4, 4, 3>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, s);
+    case 0: return op_gemm_launch<float, 1, 2, 16, 2>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, false, s);
+    case 1: return op_gemm_launch<float, 1, 4, 8, 2>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, false, s);
+    case 2: return op_gemm_launch<float, 2, 4, 4, 4>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, false, s);
+    default: return op_gemm_launch<float, 4, 4, 4, 3>(x, w, y, M, K, N, 0, 1.0f, 1.0f, 1.0f, false, s);
     }
 }
 
@@ -418,10 +419,12 @@ int hm_launch_op_gemm_w8a32(const float* x, const int8_t* q, float scale, int32_
     std::frexp(scale, &e);
     e = e - 1 < -100 ? -100 : e - 1 > 100 ? 100 : e - 1;
     const float p2 = std::ldexp(1.0f, e), mant = scale / p2 / kOpScale;
+    // the reference's weights (q - zp) * scale may lie past the float range
+    const bool past = std::isinf((float)std::max(127 - zp, 128 + zp) * scale);
     switch (op_gemm_tile(kOpTilesI8, M, K, N)) {
-    case 0: return op_gemm_launch<int8_t, 1, 2, 16, 2>(x, q, y, M, K, N, zp, p2, mant, scale, s);
-    case 1: return op_gemm_launch<int8_t, 1, 4, 8, 2>(x, q, y, M, K, N, zp, p2, mant, scale, s);
-    case 2: return op_gemm_launch<int8_t, 2, 4, 4, 4>(x, q, y, M, K, N, zp, p2, mant, scale, s);
-    default: return op_gemm_launch<int8_t, 4, 4, 4, 2>(x, q, y, M, K, N, zp, p2, mant, scale, s);
+    case 0: return op_gemm_launch<int8_t, 1, 2, 16, 2>(x, q, y, M, K, N, zp, p2, mant, scale, past, s);
+    case 1: return op_gemm_launch<int8_t, 1, 4, 8, 2>(x, q, y, M, K, N, zp, p2, mant, scale, past, s);
+    case 2: return op_gemm_launch<int8_t, 2, 4, 4, 4>(x, q, y, M, K, N, zp, p2, mant, scale, past, s);
+    default: return op_gemm_launch<int8_t, 4, 4, 4, 2>(x, q, y, M, K, N, zp, p2, mant, scale, past, s);
     }
 }

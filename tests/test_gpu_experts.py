@@ -178,6 +178,29 @@ def test_op_gemm_tiny_activations(dev):
     assert np.all(np.abs(dev.host(y) - x64 @ w64) <= (K + 32) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64)))
 
 
+def test_op_gemm_scale_past_the_range(dev):
+    """Weights (q - zp) * scale beyond the float range are infinite, as in the
+    reference's loop, however small the activations."""
+    M, K, N, zp = 20, 96, 40, -28
+    rng = np.random.default_rng(6)
+    x = (rng.standard_normal((M, K)) * 2.0 ** -60).astype(np.float32)
+    x[2, 5] = 0.0
+    q = rng.integers(-60, 60, (K, N)).astype(np.int8)
+    q[5, 3], q[7, 9], q[5, 11], q[6, 11] = 100, 127, 110, 120
+    scale = float(np.float32(2.0 ** 121))
+    y = dev.empty((M, N), np.float32)
+    _op_call(dev, dev.to(x), dev.to(q), y, scale, zp)
+    got = dev.host(y)
+    with np.errstate(all="ignore"):
+        ref = O.matmul_w8a32(x, q, scale, zp)
+    fine = np.isfinite(ref)
+    assert not fine[:, [3, 9, 11]].any() and fine[:, 20].all()
+    assert_bitexact(np.isnan(got), np.isnan(ref), "NaN outputs")
+    assert_bitexact(got[np.isinf(ref)], ref[np.isinf(ref)], "infinite outputs")
+    x64, w64 = x.astype(np.float64), (q.astype(np.float64) - zp) * scale
+    assert np.all((np.abs(got - x64 @ w64) <= (K + 32) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64)))[fine])
+
+
 def test_op_gemm_nonfinite_rows_keep_the_speed(dev):
     """Outputs that are not finite come from the matrix cores too: a call whose
     every output is infinite takes no more than ten times the finite one's time
