@@ -325,7 +325,7 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void op_gemm_kernel(
 #pragma unroll
                 for (int f = 0; f < CF; ++f) acc[rf][f] = f4{};
             const int64_t end = min(s1 * S::K, K);
-#pragma unroll 4
+#pragma clang loop unroll(disable)
             for (int64_t k0 = s0 * S::K; k0 < end; k0 += 4) {
                 const int64_t k = min(k0 + g, K - 1);  // both operands are zero past K
                 const bool in = k0 + g < K;
