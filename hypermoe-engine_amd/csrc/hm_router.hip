@@ -66,7 +66,7 @@ __device__ __forceinline__ void hm_chain64(double& acc, double p0, double p1, do
                  HM_CHAIN4(0) HM_CHAIN4(1) HM_CHAIN4(2) HM_CHAIN4(3) HM_CHAIN4(4) HM_CHAIN4(5)
                  HM_CHAIN4(6) HM_CHAIN4(7) HM_CHAIN4(8) HM_CHAIN4(9) HM_CHAIN4(10) HM_CHAIN4(11)
                  HM_CHAIN4(12) HM_CHAIN4(13) HM_CHAIN4(14) HM_CHAIN4(15)
-                 : "+v"(acc)
+                 : "+&v"(acc)
                  : "v"(p0), "v"(p1), "v"(p2), "v"(p3), "v"(1.0));
 }
 #undef HM_CHAIN4

@@ -20,7 +20,7 @@ kernel.  Loads the compiler itself tracks pass trivially (the compiler waits
 before every use, and its counts never exceed the true count of younger
 instructions), so the check covers every kernel of the file.
 
-Two further rules guard the hand-written blocks (between the compiler's
+Three further rules guard the hand-written blocks (between the compiler's
 ;;#ASMSTART and ;;#ASMEND markers):
 
 - M0.  The LDS-DMA statements set M0 themselves and name it as clobbered,
@@ -35,6 +35,9 @@ Two further rules guard the hand-written blocks (between the compiler's
   Any other vector memory instruction (another width, an AGPR destination,
   a flat or global register load, a store) is refused, since its registers
   would escape the first rule.
+- Accumulator of a chain.  The FP64 chains (csrc/hm_router.hip, hm_chain64)
+  write their accumulator at every step and read their terms until the last
+  one, so no term may share a register with the accumulator.
 """
 from __future__ import annotations
 
@@ -134,6 +137,8 @@ def _check_blocks(ins: list[list[str]], flags: list[bool]) -> list[tuple[int, st
             bad.append((i, "M0 used outside a hand-written block"))
         if in_asm and _VMEM.match(u[0]) and not _asm_vmem_ok(u):
             bad.append((i, "unrecognised vector memory instruction in a hand-written block"))
+        if in_asm and u[0].startswith("v_fmac_f64") and any(_vregs(u[1]) & _vregs(o) for o in u[2:4]):
+            bad.append((i, "a chain's accumulator is one of its terms"))
     return bad
 
 

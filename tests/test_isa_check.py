@@ -12,7 +12,7 @@ from pathlib import Path
 import pytest
 
 from hmoe import isa_check
-from hmoe.build import OBJ, _device_listing
+from hmoe.build import CSRC, OBJ, _device_listing
 
 HEAD = "k:\n"
 LOAD = "\tbuffer_load_dwordx4 v[4:7], v0, s[0:3], s4 offen\n"
@@ -102,6 +102,26 @@ def test_unrecognised_memory_forms_in_blocks_are_flagged():
     assert bad(blk("\tbuffer_load_dword v4, v0, s[0:3], s4 offen\n")) >= 1
     assert bad(blk("\tglobal_load_dwordx4 v[4:7], v[0:1], off\n")) >= 1
     assert bad(blk("\tglobal_store_dword v[0:1], v4, off\n")) >= 1
+
+
+def test_chain_accumulator_apart_from_its_terms():
+    def chain(acc, term, one):
+        steps = "".join(f"\tv_fmac_f64_dpp {acc}, {t}, {one} row_newbcast:{i} row_mask:0xf bank_mask:0xf\n"
+                        for i, t in enumerate(("v[4:5]", term)))
+        return HEAD + "\t;;#ASMSTART\n\ts_nop 4\n" + steps + "\t;;#ASMEND\n" + END
+    assert bad(chain("v[2:3]", "v[6:7]", "v[8:9]")) == 0
+    # a term, or the factor 1.0, in the accumulator's registers (whole or half)
+    assert bad(chain("v[2:3]", "v[2:3]", "v[8:9]")) >= 1
+    assert bad(chain("v[2:3]", "v[3:4]", "v[8:9]")) >= 1
+    assert bad(chain("v[2:3]", "v[6:7]", "v[2:3]")) >= 1
+
+
+def test_chain_statement_keeps_its_accumulator_apart():
+    """The compiler may place a term in the accumulator's register where both
+    hold the same value on entry, unless the operand is an early clobber."""
+    source = (CSRC / "hm_router.hip").read_text()
+    body = source[source.index("void hm_chain64("):source.index("#undef HM_CHAIN4")]
+    assert '"+&v"(acc)' in body
 
 
 @pytest.mark.parametrize("source", ["hm_gemm_mfma", "hm_router", "hm_gemm_f32_mfma"])
