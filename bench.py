@@ -450,7 +450,7 @@ def main():
             roof["traffic_detail"] = tr
         if prefill and cfg.int8:
             hw = pmc_mfma(cfg.name, {"gate_up": "ring_gemm_kernel<[0-9], false>",
-                                     "down": "ring_gemm_kernel<[0-9], true>|limb_gemm_kernel"},
+                                     "down": "ring_gemm_kernel<[0-9], true>"},
                           (args.limbs_x, args.limbs_z), q)
             if hw is not None:
                 roof["hw_mfma"] = hw

@@ -93,15 +93,6 @@ __device__ __forceinline__ int hm_wave_sum_i32(int v) {
     return v;
 }
 
-__device__ __forceinline__ unsigned long long hm_wave_max_u64(unsigned long long v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        unsigned long long o = __shfl_xor(v, m, HM_WAVE);
-        v = o > v ? o : v;
-    }
-    return v;
-}
-
 // Max / sum over each 16-lane row of the wave with DPP (quad_perm 1032,
 // quad_perm 2301, row_half_mirror, row_mirror): every lane of the row gets
 // the result.  Max and integer sums are order-free, so the result is exact.
@@ -153,20 +144,6 @@ __device__ __forceinline__ unsigned long long hm_readlane_u64(unsigned long long
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v & 0xffffffffull), l);
     const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), l);
     return ((unsigned long long)hi << 32) | lo;
-}
-__device__ __forceinline__ unsigned long long hm_wave_max_u64_dpp(unsigned long long v) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const unsigned long long o = hm_dpp_u64(v, c);
-        v = o > v ? o : v;
-    }
-    unsigned long long m = hm_readlane_u64(v, 0);
-#pragma unroll
-    for (int r = 16; r < HM_WAVE; r += 16) {
-        const unsigned long long o = hm_readlane_u64(v, r);
-        m = o > m ? o : m;
-    }
-    return m;
 }
 // Maximum of unsigned words over the wave, kept in the vector unit to the
 // end: after the row steps, row_bcast:15 hands rows 0 and 2 on to rows 1 and

@@ -21,37 +21,12 @@
 //   ring_gemm_kernel<L, true> (down): the same kernel on the grouped rows'
 //            Z digit planes and the down tiles; epilogue y -> floats.
 //   ring_gemm_ragged_kernel: both for shapes off the tile grid.
-//   limb_gemm_kernel (down, for shapes the ring does not take): 4 wave64s
-//            (one per SIMD, 512 registers: the accumulators take the
-//            AGPRs), A through an LDS ring by DMA, B straight into a
-//            register ring.
 //
-// limb_gemm_kernel, per stage of K = 128 bytes (four MFMA K steps):
-//   A  global -> LDS by 16-byte buffer loads to LDS (inline asm), 128-byte
-//      row chunks (whole cache lines), into a ring of kSA stages.  Each row's
-//      eight 16-byte chunks are stored rotated by (row >> 1) & 7, so the
-//      readers' ds_read_b128 over any 16 lanes hit 16 distinct bank groups.
-//   B  global -> VGPRs, a ring of DB stages of registers, loaded DB-1 stages
-//      ahead by loads the compiler does not track (buf_load16).
-// One vmcnt wait per stage completes both operands of the next stage.
-// Every wave issues its share of the loads of later stages between the
-// MFMAs of the current one (a wave that issues its loads in a clump stalls
-// the matrix pipe behind them).  Stages form one stream per workgroup across
-// its tiles, so the next tile's first stages load during the current tile's
-// last stages and its epilogue.  The kernel waits for its loads with
-// explicit vmcnt counts (every vector memory instruction between the awaited
-// load and the wait is counted; stores and metadata loads only add to the
-// count, which keeps the wait conservative).  A tile is BM grouped rows of
-// one expert x 256 output columns; every wave holds all BM rows and its own
-// two 32-column fragments (output columns 64 w .. +63).
-//
-// Tile order (both kernels): tiles are numbered m-tile major, column block
-// minor, and split into 8 contiguous ranges, one per XCD (workgroup i runs
-// on XCD i % 8), so the column blocks of an m-tile (sharing A rows) and the
-// m-tiles of one expert (sharing B tiles) meet in one XCD's L2.  In an
-// expert's partial last tile, the 32-row fragments past its last row skip
-// their MFMAs (down: tiles of two row fragments; gate/up: the waves whose
-// rows all lie past it).
+// Tile order: tiles are numbered m-tile major, column block minor, and split
+// into 8 contiguous ranges, one per XCD (workgroup i runs on XCD i % 8), so the
+// column blocks of an m-tile (sharing A rows) and the m-tiles of one expert
+// (sharing B tiles) meet in one XCD's L2.  In an expert's partial last tile, the
+// waves whose rows all lie past its last row skip their MFMAs.
 #include "hm_device.h"
 #include "hm_lds_dma.h"
 
@@ -61,90 +36,11 @@
 
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = 64 * kWaves;
-constexpr int kKS = 128;            // K bytes per stage
-constexpr int kKT = kKS / 32;       // MFMA K steps per stage
-constexpr int kSA = 4;              // A ring stages (LDS)
 constexpr int kXcds = 8;
 constexpr int kMaxExperts = 256;    // expert tables live in LDS
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-
-template <int L, int DB>
-struct Tile {
-    static constexpr int RF = L <= 2 ? 4 : 2;            // 32-row fragments per tile
-    static constexpr int BM = 32 * RF;                   // tile rows
-    static constexpr int NCF = 2;                        // 32-column fragments per wave
-    static constexpr int BN = 32 * NCF * kWaves;             // output columns
-    static constexpr int ASTAGE = L * BM * kKS;          // A bytes per stage
-    static constexpr int ALOADS = ASTAGE / 1024;         // wave-wide A loads per stage
-    static constexpr int APW = ALOADS / kWaves;          // ... per wave
-    static constexpr int BPW = NCF * kKT;                // B loads per wave per stage
-    static constexpr int NV = APW + BPW;                 // loads per wave per stage
-    static constexpr int NG = kKT * RF;                  // (K step, row fragment) groups per stage
-    static_assert(ALOADS % kWaves == 0 && APW <= BPW && DB >= 2 && DB <= kSA && kKT % 2 == 0,
-                  "tile shape");
-    // A stage's load items: its B loads first, then its A DMAs; item j is
-    // issued before group item_group(j) of the stage.
-    static constexpr bool item_is_a(int j) { return j >= BPW; }
-    static constexpr int item_a(int j) { return j - BPW; }
-    static constexpr int item_b(int j) { return j; }
-    static constexpr int item_group(int j) { return j * NG / NV; }
-    // the wait of a stage comes before its last K step's groups
-    static constexpr int kWaitGroup = (kKT - 1) * RF;
-    static constexpr int items_before(int g) {
-        int n = 0;
-        for (int j = 0; j < NV; ++j) n += item_group(j) < g ? 1 : 0;
-        return n;
-    }
-    static_assert(item_group(BPW - 1) < kWaitGroup, "B items precede the wait");
-    // The one wait of stage g completes both operands of stage g+1:
-    //   A(g+1): DMAs of stage g+2-kSA, the last items of that stage;
-    //   B(g+1): loads of stage g+2-DB, the first BPW items of that stage.
-    // Each count is the number of loads issued after the last awaited one
-    // (vector memory loads complete in issue order).
-    static constexpr int a_count = (kSA - 3) * NV + items_before(kWaitGroup);
-    static constexpr int b_count = (DB - 2) * NV + items_before(kWaitGroup) - BPW;
-    static constexpr int wait_count = a_count < b_count ? a_count : b_count;
-    static_assert(wait_count >= 0 && wait_count <= 63, "vmcnt");
-};
-
-// One wave-wide 16-byte buffer -> LDS load: lane l's 16 bytes from
-// rsrc + voff + soff land at lds_base + 16 l (M0 holds the wave-uniform LDS
-// base; the statement sets it itself, as dma16 does).  Loads past the
-// buffer's size return zeros instead of faulting.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff,
-                                          void* lds_base) {
-    const unsigned m0 = (unsigned)(uintptr_t)(lds_ptr_t)lds_base;
-    asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 ::"v"(voff), "s"(rsrc), "s"(soff), "s"(m0) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// One wave-wide 16-byte buffer -> VGPR load the compiler does not track:
-// it inserts no wait for the result, so the kernel's own vmcnt waits (which
-// count the DMAs too) decide when the registers are complete, and
-// publish() marks that point.  (The compiler's own waits would count only
-// the loads it knows of and so drain loads issued half as long ago as the
-// register ring allows.)  Until its wait the register must not be read,
-// copied or spilled; the build checks this on the compiled code, along every
-// control-flow path (hmoe/isa_check.py), and refuses a library that breaks it.
-__device__ __forceinline__ v4i buf_load16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff) {
-    v4i r;
-    asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen" : "=v"(r) : "v"(voff), "s"(rsrc), "s"(soff));
-    return r;
-}
-// After the vmcnt wait that completes a buf_load16: ties the value to that
-// point, so no use of it is scheduled before the wait.
-__device__ __forceinline__ void publish(v4i& r) { asm volatile("" : "+v"(r)); }
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
 
 template <int N>
 __device__ __forceinline__ void vm_wait() {
@@ -152,23 +48,9 @@ __device__ __forceinline__ void vm_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// The lane index, recomputed where it is used: derived per-lane constants
-// are then formed at their (once-per-tile) use instead of being hoisted out
-// of the tile loop, where they would occupy registers the accumulator
-// pipeline needs.
-__device__ __forceinline__ int fresh_lane() {
-    int v = (int)(threadIdx.x & 63);
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
 __device__ __forceinline__ v16i mfma32(v4i a, v4i b, v16i c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
 }
-
-// Position of 16-byte chunk c of ring row r (rotated by the row); its own
-// inverse in c.
-__device__ __forceinline__ int a_chunk_pos(int r, int c) { return c ^ ((r >> 1) & 7); }
 
 // Exclusive prefix of the m-tiles of every expert (ceil(count / bm)) into
 // prefix[0..E], prefix[E] = total.  One full wave.
@@ -224,321 +106,6 @@ __device__ __forceinline__ TileRange tile_range(int total) {
 struct TileInfo {
     int e, nrows, g0, n0;
 };
-
-// ---------------------------------------------------------------------------
-// The down projection: K = I, N = H, out = y [R x H].  A rows: the Z digit
-// planes adig (the Z layout hm_dlay_z: [K/64][L][R][64]) by grouped row;
-// ascale/adsum: their fixed-point scales [arows] and digit sums [L][arows]
-// (for non-zero zero points).
-// ---------------------------------------------------------------------------
-template <int L, int DB>
-__global__ __launch_bounds__(kThreads) void limb_gemm_kernel(
-    const int8_t* __restrict__ adig, const float* __restrict__ ascale,
-    const int32_t* __restrict__ adsum, int arows, int K, int N, int H, int I, int experts,
-    const int8_t* __restrict__ packed, const float* __restrict__ scale,
-    const int32_t* __restrict__ zp, const int32_t* __restrict__ counts,
-    const int32_t* __restrict__ offsets, int skinny, float* __restrict__ out) {
-    using T = Tile<L, DB>;
-    constexpr int RF = T::RF, BM = T::BM, BN = T::BN, NCF = T::NCF, APW = T::APW,
-                  BPW = T::BPW, NV = T::NV, ASTAGE = T::ASTAGE;
-    constexpr int MW = BM / HM_WAVE;  // 64-row metadata chunks of a tile
-    __shared__ __attribute__((aligned(1024))) int8_t ring[kSA * ASTAGE];
-    __shared__ int32_t s_prefix[kMaxExperts + 1];
-    __shared__ int32_t s_off[kMaxExperts], s_cnt[kMaxExperts];
-    __shared__ float s_sa[kMaxExperts];     // down projection scale
-    __shared__ int32_t s_za[kMaxExperts];   // and zero point
-    __shared__ __attribute__((aligned(16))) float s_as[2][BM];       // A row scale
-    __shared__ __attribute__((aligned(16))) int32_t s_ad[2][L][BM];  // A row digit sums
-
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int E = experts;
-    for (int e = tid; e < E; e += kThreads) {
-        s_cnt[e] = counts[e];
-        s_off[e] = offsets[e];
-        s_sa[e] = scale[3 * e + 2];
-        s_za[e] = zp[3 * e + 2];
-    }
-    __syncthreads();
-    if (wave == 0) tile_prefix(s_cnt, E, BM, skinny, s_prefix);
-    __syncthreads();
-    const int nbn = N / BN;
-    const TileRange tr = tile_range(s_prefix[E] * nbn);
-    if (tr.ntiles == 0) return;
-    const int nk = K / kKS;                  // stages per tile (a multiple of DB)
-    const int G = tr.ntiles * nk;            // stages of the workgroup's stream
-    const int64_t K32 = hm_pad32(K);
-
-    auto info = [&](int i) __attribute__((always_inline)) {
-        const int j = tr.jbeg + i * tr.step;
-        const int gm = j / nbn;
-        TileInfo t;
-        t.e = locate_expert(s_prefix, E, gm);
-        const int mt = gm - s_prefix[t.e];
-        t.g0 = s_off[t.e] + mt * BM;
-        t.nrows = min(BM, s_cnt[t.e] - mt * BM);
-        t.n0 = (j % nbn) * BN;
-        return t;
-    };
-    // the A rows' scales and digit sums into s_as[m], s_ad[m]
-    auto fetch_meta = [&](const TileInfo& t, int m) __attribute__((always_inline)) {
-        if (wave < MW) {
-            const int r = HM_WAVE * wave + fresh_lane();
-            const int src = t.g0 + min(r, t.nrows - 1);
-            dma4(ascale + src, &s_as[m][HM_WAVE * wave]);
-#pragma unroll
-            for (int l = 0; l < L; ++l)
-                dma4(adsum + (int64_t)l * arows + src, &s_ad[m][l][HM_WAVE * wave]);
-        }
-    };
-
-    // ---- load sources of a tile (buffer resources: wave-uniform bases,
-    // 32-bit per-lane offsets)
-    // A: load unit u = wave + kWaves i covers ring rows 8u .. 8u+7 (limb-major
-    // [L][BM], 128 bytes a row); lane: row 8u + lane/8, ring position lane%8,
-    // which holds chunk a_chunk_pos(row, lane%8) of the row's stage: in the Z
-    // layout, 16-byte piece c of stage ks lies in 64-byte chunk 2 ks + c/4
-    // (the stage's uniform offset ks * astep, astep = 2 L arows 64).
-    const __amdgpu_buffer_rsrc_t arsrc = buffer_rsrc(adig, (uint32_t)((int64_t)L * arows * K));
-    const uint32_t astep = (uint32_t)(2 * 64 * (int64_t)L * arows);
-    uint32_t aoff[APW];
-    auto make_asrc = [&](const TileInfo& t) __attribute__((always_inline)) {
-        const int ln = fresh_lane();
-#pragma unroll
-        for (int i = 0; i < APW; ++i) {
-            const int q = 8 * (wave + kWaves * i) + (ln >> 3);
-            const int l = q / BM, r = q % BM;
-            const int c = a_chunk_pos(r, ln & 7);
-            const int row = t.g0 + min(r, t.nrows - 1);
-            aoff[i] = (uint32_t)((((int64_t)(c >> 2) * L + l) * arows + row) * 64 + 16 * (c & 3));
-        }
-    };
-    // B: the tile's expert as one buffer; fragment f's K tiles are
-    // contiguous from boff[f] (uniform) + 16 lane
-    __amdgpu_buffer_rsrc_t brsrc;
-    int boff[NCF];
-    const uint32_t blane = 16u * (uint32_t)lane;
-    auto make_bsrc = [&](const TileInfo& t) __attribute__((always_inline)) {
-        brsrc = buffer_rsrc(packed + hm_proj_offset(t.e, 0, H, I), (uint32_t)(3 * hm_proj_bytes(H, I)));
-#pragma unroll
-        for (int f = 0; f < NCF; ++f) {
-            const int cb = t.n0 / 32 + NCF * wave + f;
-            boff[f] = (int)(2 * hm_proj_bytes(H, I) + (int64_t)cb * (K32 / 32) * 1024);
-        }
-    };
-    auto issue_a = [&](int i, int stage, int ks) __attribute__((always_inline)) {
-        dma16_buf(arsrc, aoff[i], (uint32_t)ks * astep,
-                  ring + (stage % kSA) * ASTAGE + (wave + kWaves * i) * 1024);
-    };
-    v4i bq[DB][NCF][kKT];
-    auto publish_slot = [&](int slot) __attribute__((always_inline)) {
-#pragma unroll
-        for (int f = 0; f < NCF; ++f)
-#pragma unroll
-            for (int kt = 0; kt < kKT; ++kt) publish(bq[slot][f][kt]);
-    };
-    auto load_b = [&](int slot, int j, int ks) __attribute__((always_inline)) {
-        const int f = j / kKT, kt = j % kKT;
-        bq[slot][f][kt] = buf_load16(brsrc, blane, (uint32_t)(boff[f] + (ks * kKT + kt) * 1024));
-    };
-
-    // ---- A fragment reads: the L limb planes of every row fragment of one K
-    // step, read a K step ahead into alternating buffers
-    v4i fa[2][L][RF];
-    auto read_a = [&](int buf, int stage, int kt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int rf = 0; rf < RF; ++rf) {
-            const int r = 32 * rf + (lane & 31);
-            const int c = 2 * kt + (lane >> 5);
-            const int8_t* base = ring + (stage % kSA) * ASTAGE + r * kKS + 16 * a_chunk_pos(r, c);
-#pragma unroll
-            for (int l = 0; l < L; ++l) fa[buf][l][rf] = *reinterpret_cast<const v4i*>(base + l * BM * kKS);
-        }
-    };
-
-    v16i acc[L][RF][NCF];
-
-    // ---- stream prologue: tile 0's row metadata, the A of stages 0 .. kSA-2
-    // and the B of stages 0 .. DB-2 (all of tile 0: nk >= kSA)
-    TileInfo cur = info(0);
-    fetch_meta(cur, 0);
-    make_asrc(cur);
-    make_bsrc(cur);
-#pragma unroll
-    for (int s = 0; s < kSA - 1; ++s)
-#pragma unroll
-        for (int i = 0; i < APW; ++i) issue_a(i, s, s);
-#pragma unroll
-    for (int s = 0; s < DB - 1; ++s)
-#pragma unroll
-        for (int j = 0; j < BPW; ++j) load_b(s, j, s);
-    // A(0) landed and published; its first K step's fragments
-    vm_wait<0>();
-    lds_barrier();
-#pragma unroll
-    for (int s = 0; s < DB - 1; ++s) publish_slot(s);
-    read_a(0, 0, 0);
-
-    int m = 0;
-    int g = 0;  // stage index in the stream
-    for (int i = 0; i < tr.ntiles; ++i) {
-        const bool has_next = i + 1 < tr.ntiles;
-        TileInfo nxt = cur;
-        if (has_next) nxt = info(i + 1);
-        const int mn = m ^ 1;
-        // the stage items load kSA-1 (A) and DB-1 (B) stages ahead: the next
-        // tile's sources switch in at these stages of this tile.  Past the
-        // end of the stream the items repeat this tile's loads into slots no
-        // stage reads (no branch in the load pattern, and the vmcnt counts
-        // hold everywhere).
-        const int ka_switch = nk - (kSA - 1), kb_switch = nk - (DB - 1);
-
-        // One stage: K steps kt = 0..kKT-1, each the L * RF * NCF MFMAs with
-        // the stage's load items spread over its row-fragment groups.  The
-        // wait for A(g+1) and the barrier that publishes it come before the
-        // last K step, whose MFMAs overlap the reads of the next stage's first
-        // K step.
-        auto stage = [&](int ks, auto phase, auto first) __attribute__((always_inline)) {
-            constexpr int PH = decltype(phase)::value;
-            constexpr int WS = PH;                   // B ring slot this stage uses
-            constexpr int WL = (PH + DB - 1) % DB;   // slot its B items fill
-            const int ta = g + kSA - 1;              // stage its A items load
-            const int ksa = ks + kSA - 1 < nk ? ks + kSA - 1 : ks + kSA - 1 - nk;
-            const int ksb = ks + DB - 1 < nk ? ks + DB - 1 : ks + DB - 1 - nk;
-            if (ks == ka_switch && has_next) {
-                make_asrc(nxt);
-                fetch_meta(nxt, mn);
-            }
-            if (ks == kb_switch && has_next) make_bsrc(nxt);
-#pragma unroll
-            for (int kt = 0; kt < kKT; ++kt) {
-                if (kt == kKT - 1) {
-                    // A(g+1) and B(g+1) have landed (issued by stages
-                    // g+2-kSA and g+2-DB, or by the prologue, which ends with
-                    // a full wait); the barrier publishes A(g+1)
-                    vm_wait<T::wait_count>();
-                    lds_barrier();
-                    publish_slot((PH + 1) % DB);
-                }
-                const int rb = kt & 1;  // kKT is even: every stage starts on buffer 0
-                // the next K step's fragments (after the last: the next
-                // stage's first, published by the barrier above)
-                if (kt + 1 < kKT) read_a(rb ^ 1, g, kt + 1);
-                else read_a(rb ^ 1, g + 1, 0);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int rf = 0; rf < RF; ++rf) {
-                    const int gi = kt * RF + rf;
-#pragma unroll
-                    for (int j = 0; j < NV; ++j) {
-                        if (T::item_group(j) == gi) {
-                            __builtin_amdgcn_sched_barrier(0);
-                            if (T::item_is_a(j)) issue_a(T::item_a(j), ta, ksa);
-                            else load_b(WL, T::item_b(j), ksb);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-                    // row fragments past the tile's last row (an expert's
-                    // partial last tile) skip their MFMAs; the epilogue skips
-                    // their accumulators.  Only with two row fragments: with
-                    // four, the branches split the accumulator ranges and the
-                    // allocator spills them.
-                    if (RF <= 2 ? (rf == 0 || 32 * rf < cur.nrows) : true) {
-#pragma unroll
-                        for (int l = 0; l < L; ++l)
-#pragma unroll
-                            for (int f = 0; f < NCF; ++f) {
-                                if (decltype(first)::value && kt == 0)
-                                    acc[l][rf][f] = mfma32(fa[rb][l][rf], bq[WS][f][kt], v16i{});
-                                else
-                                    acc[l][rf][f] = mfma32(fa[rb][l][rf], bq[WS][f][kt], acc[l][rf][f]);
-                            }
-                    }
-                }
-            }
-            ++g;
-        };
-
-        // stages in groups of DB (static B ring slots); the first stage
-        // starts the accumulators
-        stage(0, std::integral_constant<int, 0>{}, std::true_type{});
-        if constexpr (DB > 1) stage(1, std::integral_constant<int, 1 % DB>{}, std::false_type{});
-        if constexpr (DB > 2) stage(2, std::integral_constant<int, 2 % DB>{}, std::false_type{});
-        if constexpr (DB > 3) stage(3, std::integral_constant<int, 3 % DB>{}, std::false_type{});
-#pragma clang loop unroll(disable)
-        for (int ks = DB; ks < nk; ks += DB) {
-            stage(ks, std::integral_constant<int, 0>{}, std::false_type{});
-            if constexpr (DB > 1) stage(ks + 1, std::integral_constant<int, 1 % DB>{}, std::false_type{});
-            if constexpr (DB > 2) stage(ks + 2, std::integral_constant<int, 2 % DB>{}, std::false_type{});
-            if constexpr (DB > 3) stage(ks + 3, std::integral_constant<int, 3 % DB>{}, std::false_type{});
-        }
-
-        // ---- epilogue (the next tile's first stages are in flight).  The
-        // zero-point correction is chosen once per tile (uniform), so no
-        // per-element test drags integer multiplies into the common case.
-        auto epilogue = [&](auto with_zp) __attribute__((always_inline)) {
-            constexpr bool ZP = decltype(with_zp)::value;
-            const int e = cur.e;
-            const float sa = s_sa[e];
-            const int za = s_za[e];
-            // out [R x N], the wave's two fragments side by side.  The
-            // lane's row within a row quad (0 or 4) and its column;
-            // everything else is uniform per (row fragment, quad).
-            const int64_t ldo = N;
-            const int fstride = 32;
-            const int lrow = 4 * (lane >> 5);
-            float* obase = out + (int64_t)cur.g0 * ldo + cur.n0 + 64 * wave +
-                           (int64_t)lrow * ldo + (lane & 31);
-#pragma unroll
-            for (int rf = 0; rf < RF; ++rf) {
-                if (32 * rf >= cur.nrows) continue;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int r0 = 32 * rf + 8 * q;          // uniform
-                    const int nlive = cur.nrows - r0 - lrow;  // rows t4 < nlive are live
-                    const float4 as4 = *reinterpret_cast<const float4*>(&s_as[m][r0 + lrow]);
-                    int4 ad4[L];
-                    if constexpr (ZP) {
-#pragma unroll
-                        for (int l = 0; l < L; ++l) ad4[l] = *reinterpret_cast<const int4*>(&s_ad[m][l][r0 + lrow]);
-                    }
-                    float* o = obase + (int64_t)r0 * ldo;
-#pragma unroll
-                    for (int t4 = 0; t4 < 4; ++t4) {
-                        const int v = 4 * q + t4;
-                        const float asc = t4 == 0 ? as4.x : t4 == 1 ? as4.y : t4 == 2 ? as4.z : as4.w;
-                        if (t4 < nlive) {
-#pragma unroll
-                            for (int f = 0; f < NCF; ++f) {
-                                int p[L];
-#pragma unroll
-                                for (int l = 0; l < L; ++l) {
-                                    p[l] = acc[l][rf][f][v];
-                                    if constexpr (ZP) {
-                                        const int ds = t4 == 0 ? ad4[l].x : t4 == 1 ? ad4[l].y : t4 == 2 ? ad4[l].z : ad4[l].w;
-                                        p[l] -= za * ds;
-                                    }
-                                }
-                                const float wsc = __fmul_rn(asc, sa);
-                                o[(int64_t)t4 * ldo + fstride * f] = __fmul_rn(hm_recombine(p, L), wsc);
-                            }
-                        }
-                    }
-                    // one (row fragment, row quad) at a time: the scheduler
-                    // would otherwise start every group's accumulator reads
-                    // at once and spill
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-        };
-        const bool zpt = s_za[cur.e] != 0;
-        if (zpt) epilogue(std::true_type{});
-        else epilogue(std::false_type{});
-        m = mn;
-        cur = nxt;
-    }
-    vm_wait<0>();
-}
 
 // ===========================================================================
 // Skinny groups: bounded split-K.  An expert with at most kSkinnyRows = 32
@@ -750,58 +317,6 @@ int persistent_grid() {
     }
     const int g = cached[dev] / kXcds * kXcds;
     return g < kXcds ? kXcds : g;
-}
-
-// B ring depth for nk stages per tile: the largest of 4, 3, 2 dividing nk.
-int ring_depth(int64_t nk) { return nk % 4 == 0 ? 4 : nk % 3 == 0 ? 3 : nk % 2 == 0 ? 2 : 0; }
-
-bool shape_ok(int64_t K, int64_t N, int64_t E, int32_t limbs) {
-    // |P_l| <= K * 128 * 255 < 2^31 keeps every limb partial exact: K <= 65536
-    if (limbs < 1 || limbs > 3 || E < 1 || E > kMaxExperts || K > 65536 || N > (1 << 20))
-        return false;
-    if (K % kKS != 0) return false;
-    const int64_t nk = K / kKS;
-    return nk >= kSA && ring_depth(nk) != 0 && N % (64 * kWaves) == 0;
-}
-
-template <int L, int DB>
-int launch(const hm_layer* layer, const int8_t* adig, const float* ascale, const int32_t* adsum,
-           int64_t arows, const int32_t* counts, const int32_t* offsets, int skinny, float* out,
-           hipStream_t stream) {
-    const int64_t H = layer->hidden, I = layer->intermediate;
-    const int64_t K = I, N = H;
-    // buffer offsets are 32-bit: the digit planes and one expert's tiles
-    if ((int64_t)L * arows * K > INT_MAX || 3 * hm_proj_bytes(H, I) > INT_MAX || arows > INT_MAX)
-        return HM_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((limb_gemm_kernel<L, DB>), dim3((unsigned)persistent_grid()), dim3(kThreads), 0,
-                       stream, adig, ascale, adsum, (int)arows, (int)K, (int)N, (int)H, (int)I,
-                       (int)layer->experts, static_cast<const int8_t*>(layer->packed), layer->scale,
-                       layer->zero_point, counts, offsets, skinny, out);
-    HM_LAUNCHED();
-    return HM_OK;
-}
-
-template <int L>
-int launch_l(const hm_layer* layer, const int8_t* adig, const float* ascale,
-             const int32_t* adsum, int64_t arows, const int32_t* counts, const int32_t* offsets,
-             float* out, bool split_k, hipStream_t stream) {
-    if (!shape_ok(layer->intermediate, layer->hidden, layer->experts, L) ||
-        ring_depth(layer->intermediate / kKS) == 0)
-        return HM_ERR_UNSUPPORTED;
-    // skinny groups (split K, when asked for), then the tiles of the others
-    const bool sk = split_k && skinny_ok(layer->intermediate, layer->hidden, L, false);
-    if (sk) {
-        const int rc = launch_skinny<L, false>(layer, adig, ascale, adsum, arows, nullptr, counts,
-                                               offsets, out, stream, false);
-        if (rc) return rc;
-    }
-    const int skinny = sk ? kSkinnyRows : 0;
-    switch (ring_depth(layer->intermediate / kKS)) {
-    case 4: return launch<L, 4>(layer, adig, ascale, adsum, arows, counts, offsets, skinny, out, stream);
-    case 3: return launch<L, 3>(layer, adig, ascale, adsum, arows, counts, offsets, skinny, out, stream);
-    case 2: return launch<L, 2>(layer, adig, ascale, adsum, arows, counts, offsets, skinny, out, stream);
-    default: return HM_ERR_UNSUPPORTED;
-    }
 }
 
 // ===========================================================================
@@ -1298,14 +813,12 @@ bool ring_ok(int64_t K, int64_t N, int64_t E, int32_t limbs) {
 bool ring_aligned(int64_t K, int64_t N, int64_t cols) { return K % kGuKB == 0 && N % cols == 0; }
 
 // Down: skinny groups (split K, when asked for), then the tiles of the
-// others on the ring kernel, or on limb_gemm_kernel where the ring's shape
-// conditions do not hold.
+// others.
 template <int L>
 int launch_down(const hm_layer* layer, const int8_t* zdig, const float* zscale,
                 const int32_t* zdsum, int64_t R, const int32_t* counts, const int32_t* offsets,
                 float* y, bool split_k, hipStream_t stream) {
-    if (!ring_ok(layer->intermediate, layer->hidden, layer->experts, L))
-        return launch_l<L>(layer, zdig, zscale, zdsum, R, counts, offsets, y, split_k, stream);
+    if (!ring_ok(layer->intermediate, layer->hidden, layer->experts, L)) return HM_ERR_UNSUPPORTED;
     const bool sk = split_k && skinny_ok(layer->intermediate, layer->hidden, L, false);
     if (sk) {
         const int rc = launch_skinny<L, false>(layer, zdig, zscale, zdsum, R, nullptr, counts,
@@ -1360,7 +873,7 @@ bool hm_mfma_gateup_ok(int64_t H, int64_t I, int64_t E, int32_t limbs) {
 }
 
 bool hm_mfma_down_ok(int64_t H, int64_t I, int64_t E, int32_t limbs) {
-    return ring_ok(I, H, E, limbs) || shape_ok(I, H, E, limbs);
+    return ring_ok(I, H, E, limbs);
 }
 
 // gu [R x 2I]: the gate and up values of every grouped row (X digits in the

@@ -10,12 +10,12 @@ tree is mounted) oracle/_ref/libhm_ref.so.
 
 Every HIP translation unit is built with -ffp-contract=off (FMAs only where a
 kernel asks for one explicitly) and with packed FP32 instructions disabled.
-Sources with hand-written memory statements (CHECKED_SOURCES: loads the
-compiler does not track, LDS-DMA loads that set M0) are assembled from a
-saved listing that hmoe.isa_check verifies first: no register of an
-untracked load is touched before a wait completes it, the compiler's own
-code leaves M0 alone, and the hand-written blocks hold only the memory
-forms the check understands.
+Sources with hand-written memory statements (CHECKED_SOURCES: LDS-DMA loads
+that set M0) are assembled from a saved listing that hmoe.isa_check verifies
+first: the compiler's own code leaves M0 alone, the hand-written blocks hold
+only the memory forms the check understands, an FP64 chain's accumulator is
+none of its terms, and no register of an untracked load is touched before a
+wait completes it.
 """
 from __future__ import annotations
 
@@ -50,8 +50,7 @@ KERNEL_SOURCES = ["hm_runtime.hip", "hm_router.hip", "hm_gemm.hip", "hm_gemm_mfm
 SOURCE_FLAGS = {"hm_router.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                 "hm_gemm_f32_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                 "hm_op_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
-# Sources with hand-written memory statements: register loads the compiler
-# does not track (hm_gemm_mfma.hip) and LDS-DMA loads that set M0 (all three).
+# Sources with hand-written memory statements: LDS-DMA loads that set M0.
 CHECKED_SOURCES = {"hm_gemm_mfma.hip", "hm_router.hip", "hm_gemm_f32_mfma.hip"}
 HOST_SOURCES = ["hip_backend.cpp", "hip_tensor_backend.cpp", "moe_block.cpp", "artefact.cpp"]
 

@@ -1,13 +1,14 @@
 """Static check of compiled gfx950 code: no register of an untracked load is
 touched before a wait that completes the load.
 
-The grouped INT8 GEMM (csrc/hm_gemm_mfma.hip) loads its B fragments with
-inline-asm buffer loads the compiler does not track, so the compiler inserts
-no wait for them and the kernel's own `s_waitcnt vmcnt(N)` statements decide
-when the registers are complete.  If register allocation ever copied,
+A register load written as inline asm is one the compiler does not track: it
+inserts no wait for it, and the kernel's own `s_waitcnt vmcnt(N)` statements
+decide when the register is complete.  If register allocation ever copied,
 spilled or read such a register before that wait, the kernel would compute
-with stale data and no test could be relied on to notice.  This module reads
-the assembly the compiler produced for the object and proves the contrary.
+with stale data and no test could be relied on to notice.  (The kernels' asm
+loads go to LDS; a register form that is added must pass here.)  This module
+reads the assembly the compiler produced for the object and proves the
+contrary.
 
 For every `buffer_load_dwordx4 v[...]` that writes VGPRs (not the LDS
 variants, which write no registers), it follows every control-flow path from

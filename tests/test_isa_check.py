@@ -137,5 +137,5 @@ def test_built_gemm_listing_is_clean():
     if not listing.exists():
         pytest.skip("no saved listing (library not built here)")
     text = Path(listing).read_text()
-    assert "limb_gemm_kernel" in text
+    assert "ring_gemm_kernel" in text
     assert isa_check.check_text(text) == []
