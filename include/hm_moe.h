@@ -74,9 +74,10 @@ typedef enum hm_status {
 #define HM_GEMV_MAX_TOKENS 16
 #define HM_GEMV_MAX_PAIRS 64
 /* Execution flag for hm_router_topk / hm_moe_block_forward: every router
- * logit is computed with the reference's sequential FP64 chain instead of
- * certifying the parallel sums (the results are identical; the flag
- * exercises the fallback). */
+ * logit of a decode batch (up to 16 tokens) is computed with the reference's
+ * sequential FP64 chain instead of certifying the parallel sums (the results
+ * are identical; the flag exercises the fallback).  Larger batches run the
+ * chains with and without it. */
 #define HM_EXEC_ROUTE_SEQUENTIAL 0x400u
 /* Execution flag for hm_moe_block_forward: INT8 prefill experts with at most
  * 32 grouped rows take the bounded split-K GEMM (K split over a workgroup's

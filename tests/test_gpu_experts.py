@@ -624,7 +624,7 @@ def test_block_fp32_split_tiles(dev, T, H, E, I, k, skew):
     """FP32 experts on the split bf16 tiles: fragment and tile edges (16, 64, 65
     rows of an expert, one K stage of slack, fewer tiles than XCDs).  An expert
     output is two chained sums: within (H + I + 64) 2^-22 of the absolute sums
-    (a product's left-out parts are below 2^-21, each FP32 addition 2^-24)."""
+    (a product's left-out parts are below 2^-32, each FP32 addition 2^-24)."""
     print(f"[gpu] fp32 split T={T} H={H} E={E} I={I}", flush=True)
     payload, scale, zp, h, w = _layer_inputs(5 + T, T, H, E, I, False, skew=skew)
     block = MoEBlock(DeviceExpertLayer(payload, scale, zp, H, I), k)
