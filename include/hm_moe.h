@@ -170,8 +170,8 @@ int hm_gather_rows(const float* in, const int32_t* rows, int64_t count,
  * (cooperative): the terms x (q - zp) exactly, summed in FP32 in another,
  * fixed order, times the scale: within (K + 32) 2^-24 sum_k |x w| of the exact
  * sum, as the loop is within K 2^-24 of that, so the two differ by up to both
- * (on the reference's own test inputs by less than 1e-5 + 1e-5|ref|).  Terms,
- * sums and scales past the float range give what the loop gives.
+ * (on the reference's own test inputs by less than 1e-5 + 1e-5|ref|).  Non-finite
+ * activations and weights past the float range give what the loop gives.
  * The plan (hm_plan_int8_gemm) is the reference's: its partition and block
  * counts and the scratch it asks of the caller are part of the interface,
  * though the cooperative kernel splits K inside a workgroup and leaves the
