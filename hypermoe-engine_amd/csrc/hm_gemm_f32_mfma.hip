@@ -40,8 +40,9 @@
 // fragments and no wave waits for another.  K moves in stages of 32 floats
 // through a 2-slot LDS ring filled by 16-byte direct loads (global_load_lds), so
 // that three workgroups fit a CU: they cover each other's waits better than a
-// third slot does (gate/up 302 us; three slots, two workgroups 340).  Lane (g, i) = (lane/16, lane%16) supplies row or
-// column i, k = 8 g .. 8 g + 7 of the stage.  Rows of a stage are 128 bytes; the
+// third slot does (gate/up, six products: 302 us; three slots, two workgroups
+// 340).  Lane (g, i) = (lane/16, lane%16) supplies row or column i, k = 8 g ..
+// 8 g + 7 of the stage.  Rows of a stage are 128 bytes; the
 // 16-byte chunk c of row r is stored at slot c ^ (r % 8), which spreads a
 // reader's rows over the LDS banks.  Tiles are numbered row tile major, column
 // block minor, in eight contiguous ranges, one per XCD (workgroup i runs on XCD
