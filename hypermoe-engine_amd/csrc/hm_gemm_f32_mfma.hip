@@ -9,13 +9,13 @@
 // of parts other than the two last ones': each exact, what is left out below
 // 2^-32 |x w|, and the sums in FP32.  A single product is thus rounded once, as
 // an FP32 matrix instruction rounds it (six products, without the second part
-// times the third, leave out up to 2^-21 |x w|).  Long sums have a smaller error against 64-bit sums than
-// those of FP32 matrix instructions on the whole values (an expert's output at
-// K = 2048, 768: 4.6e-7 against 1.3e-6), as these round once per two k, the
-// split ones' leading sums once per 32.  The reference sums each output
-// sequentially in FP32: the results are within the FP32 path's 1e-3 of it, not
-// bit-identical (as the FMA tiles in hm_gemm.hip, which remain for other
-// shapes).  An operand that is not finite gives NaN parts, one of 2^112 and
+// times the third, leave out up to 2^-21 |x w|).  Long sums have a smaller error
+// against 64-bit sums than those of FP32 matrix instructions on the whole values
+// (an expert's output at K = 2048, 768: 4.6e-7 against 1.3e-6), as these round
+// once per two k, the split ones' leading sums once per 32.  The reference sums
+// each output sequentially in FP32: the results are within the FP32 path's 1e-3
+// of it, not bit-identical (as the FMA tiles in hm_gemm.hip, which remain for
+// other shapes).  An operand that is not finite gives NaN parts, one of 2^112 and
 // more or a sum of 2^96 and more infinite ones; a tile with such a sum is
 // summed again on FP32 matrix instructions (v_mfma_f32_16x16x4_f32), which give
 // those outputs what their operands have (512 tokens, 8 experts top-2, H = 1024,
@@ -42,12 +42,11 @@
 // that three workgroups fit a CU: they cover each other's waits better than a
 // third slot does (gate/up, six products: 302 us; three slots, two workgroups
 // 340).  Lane (g, i) = (lane/16, lane%16) supplies row or column i, k = 8 g ..
-// 8 g + 7 of the stage.  Rows of a stage are 128 bytes; the
-// 16-byte chunk c of row r is stored at slot c ^ (r % 8), which spreads a
-// reader's rows over the LDS banks.  Tiles are numbered row tile major, column
-// block minor, in eight contiguous ranges, one per XCD (workgroup i runs on XCD
-// i % 8): the row tiles of one expert read its weights at about the same time
-// from one L2.
+// 8 g + 7 of the stage.  Rows of a stage are 128 bytes; the 16-byte chunk c of
+// row r is stored at slot c ^ (r % 8), which spreads a reader's rows over the LDS
+// banks.  Tiles are numbered row tile major, column block minor, in eight
+// contiguous ranges, one per XCD (workgroup i runs on XCD i % 8): the row tiles
+// of one expert read its weights at about the same time from one L2.
 #include "hm_device.h"
 #include "hm_lds_dma.h"
 

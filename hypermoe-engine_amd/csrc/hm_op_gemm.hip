@@ -112,8 +112,9 @@ __device__ __forceinline__ void op_split(const f4 (&x)[2], bf8 (&p)[3]) {
 }
 
 // x [M x K], w [K x N], y [M x N].  WT = int8_t: y = mant * (the sum of 2^16 x
-// with p2-scaled weights), scale = 2^16 mant p2; zp the zero point.  WT = float: the
-// last five arguments are not read.
+// with p2-scaled weights), scale = 2^16 mant p2; zp the zero point; past: some
+// (q - zp) * scale may be infinite.  WT = float: the last five arguments are not
+// read.
 template <typename WT, int RF, int CF, int NW, int D>
 __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void op_gemm_kernel(
     const float* __restrict__ x, const WT* __restrict__ w, float* __restrict__ y, int64_t M,
@@ -280,9 +281,8 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 4 : 2) void op_gemm_kernel(
             multiply(st);
         }
         // D of a 16 x 16 fragment: lane (g, i) holds rows 4 g .. 4 g + 3 of
-        // column i
+        // column i.  AGAIN: only the outputs that are not finite yet, or all.
         ++round;
-        // (AGAIN: only the outputs that are not finite yet, or all)
         auto finish = [&](auto again, bool all) __attribute__((always_inline)) {
             constexpr bool AGAIN = decltype(again)::value;
 #pragma unroll
